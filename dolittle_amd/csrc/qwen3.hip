@@ -38,6 +38,7 @@
 #include "dl_device.h"
 #include "dl_internal.h"
 #include "dl_synth.h"
+#include "exact_mfma.h"
 #include "gemv.h"
 #include "heads.h"
 #include "nla.h"
@@ -521,6 +522,9 @@ struct AttnArgs {
   // sequences at one position (decode), 1 when they are consecutive
   // positions of one sequence (cache_seq_stride 0, chunked prompt pass).
   int pos_step;
+  // The output rows in P16 order, for the many-row exact O projection (the
+  // row-block kernels only).
+  int permuted_out;
 };
 
 
@@ -1493,7 +1497,8 @@ __global__ __launch_bounds__(kPwThreads) void k_attn_pv_block(AttnArgs a, int ro
       if (rr < n) {
 #pragma unroll
         for (int i = 0; i < kPbFeat; ++i)
-          a.att[static_cast<uint64_t>(rb + rr) * a.q_heads * kHeadDim + (g * group + hl) * kHeadDim + f0 + i] =
+          a.att[static_cast<uint64_t>(rb + rr) * a.q_heads * kHeadDim + (g * group + hl) * kHeadDim +
+                (a.permuted_out ? static_cast<int>(prefill::permuted(f0 + i, 16)) : f0 + i)] =
               bf16_bits(acc[rr][i] + second[rr][i][lane]);
       }
   }
@@ -2471,43 +2476,27 @@ __global__ __launch_bounds__(gemv_waves(B) * 64) void k_gateup(GateUpArgs a) {
 // ---------------------------------------------- exact GEMM over many rows
 // The projections of the chunked prompt pass when a chunk holds many rows
 // (positions of one sequence).  Every output is the same P-partial FMA chain
-// and upper-into-lower merge as in the GEMV kernels (projection.cu:139-482):
-// partial t of output f is the FMA chain over inputs t, t + P, ... in
-// ascending order.  Only the assignment of chains to lanes differs: lane
-// (g, t) of a wavefront owns partial t of kXgFeat consecutive outputs for
-// kXgPos rows, so each staged input feeds kXgFeat FMAs and each widened
-// weight kXgPos, and the weights are read once per kXgRows rows instead of
-// once per step row.
+// and upper-into-lower merge as in the GEMV kernels (projection.cu:139-482),
+// run on the FP32 matrix cores (exact_mfma.h).
 //
-// Workgroup: 8 wavefronts = kXgWN output blocks x kXgWP row blocks, tile
-// kXgWN * (64 / P) * kXgFeat outputs x kXgRows rows.  The rows' inputs pass
-// through LDS kXgChunk inputs at a time as FP32 in the GEMV's staged layout
-// (partial-major rows padded by kXsPad floats, so the P lanes of a read hit
-// distinct banks); the next pass's inputs are loaded into registers while
-// the current one is multiplied.  The weights come straight from memory in
-// the packed layout, one 8-element step ahead.  Workgroups that share
-// weights (same blockIdx.x) land on one XCD when gridDim.x is a multiple of
-// 8, so its L2 serves the weights to the row blocks.
-constexpr int kXgThreads = 512;
-constexpr int kXgWN = 4, kXgWP = 2;
-constexpr int kXgFeat = 4;                  // outputs per lane (one P = 16 tile, two P = 32 tiles)
-constexpr int kXgPos = 16;                  // rows per lane
-constexpr int kXgRows = kXgWP * kXgPos;     // rows per workgroup
-constexpr int kXgChunk = 1024;              // inputs staged per pass
-constexpr int kXgMinRows = 16;              // fewer rows run through the batched GEMVs
-
+// Bound: the FP32 MFMA rate with the operands' widening (no overlap).  The
+// Qwen3-8B block's projections of 512 rows take 1.70 ms (57-60 T FMA/s) where
+// the vector-ALU form (16 rows and 4 outputs per lane, inputs as FP32 in LDS)
+// took 3.4 (28-32 T FMA/s); a tile's (outputs + rows) x 8 P inputs per stage
+// are 12 to 16 bytes per clock and compute unit from L2.
 enum XgEpilogue : int {
   kXgQ = 0,         // out[b][f] = BF16(acc): Q rows
   kXgKV = 1,        // K rows (f < kw) to out[b][f], V rows to the transposed cache column of row b
-  kXgResidual = 2,  // residual_store (O and down)
+  kXgResidual = 2,  // the residual update of residual_store (O and down)
   kXgGateUp = 3,    // interleaved [g 2j, g 2j+1, u 2j, u 2j+1] -> SiLU(g) * u, P32-permuted act rows
 };
+constexpr int kXgMinRows = 16;  // fewer rows run through the batched GEMVs
 
 struct XgemmArgs {
   const Control* ctl;
-  const uint16_t* x;     // [B][K] BF16 input rows: P-permuted (`permuted`) or natural order
+  const uint16_t* x;     // [B][K] BF16 input rows, P-permuted
   const u32x4* w;        // packed rows with P partials
-  int B, N, K, permuted;
+  int B, N, K;
   uint16_t* out;         // kXgQ [B][N]; kXgKV k rows [B][kw]; kXgGateUp act [B][N / 2]
   uint16_t* v_cache;     // kXgKV: V^T of this layer; row b's column is position + b * v_stride
   uint64_t v_stride;
@@ -2515,173 +2504,78 @@ struct XgemmArgs {
   ResidualArgs res;      // kXgResidual
 };
 
-__host__ __device__ constexpr size_t xgemm_lds(int P) {
-  return size_t(kXgRows) * P * (kXgChunk / P + kXsPad) * sizeof(float);
+__device__ __forceinline__ u32x2 pack4(const float (&v)[4]) {
+  return u32x2{bf16_bits(v[0]) | (static_cast<uint32_t>(bf16_bits(v[1])) << 16),
+               bf16_bits(v[2]) | (static_cast<uint32_t>(bf16_bits(v[3])) << 16)};
 }
 
-template <int P, int EPI>
-__global__ __launch_bounds__(kXgThreads) void k_xgemm(XgemmArgs a) {
-  constexpr int G = 64 / P;                    // lane groups of a wavefront
-  constexpr int RW = 64 / P;                   // outputs per packed tile
-  constexpr int WF = G * kXgFeat;              // outputs per wavefront
-  constexpr int TF = kXgWN * WF;               // outputs per workgroup
-  constexpr int stride = kXgChunk / P + kXsPad;
-  constexpr int row_floats = P * stride;       // staged floats per row
-  constexpr int steps = kXgChunk / (8 * P);    // 8-element chain steps per pass
-  constexpr int kPieces = kXgRows * kXgChunk / 8 / kXgThreads;  // 16-byte input pieces per thread per pass
-  static_assert(kXgFeat % RW == 0 || RW % kXgFeat == 0, "whole tiles per lane");
-  static_assert(kXgWN * kXgWP * 64 == kXgThreads, "one wavefront per (output block, row block)");
-  extern __shared__ float xs[];                // [kXgRows][P][stride]
+template <class T, int EPI>
+__global__ __launch_bounds__(exact::kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_xgemm(XgemmArgs a) {
+  constexpr int P = T::P, RW = 64 / P;
   if (!a.ctl->active) return;
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int g = lane / P, t = lane % P;
-  const int f0 = blockIdx.x * TF + (wave % kXgWN) * WF + g * kXgFeat;  // first output of this lane
-  const int b0 = blockIdx.y * kXgRows;                                 // first row of the workgroup
-  const int pb = (wave / kXgWN) * kXgPos;                              // first row of this lane in the tile
-  const int S = a.K / (8 * P), passes = a.K / kXgChunk;
+  // Workgroups are dealt to the XCDs round-robin: XCD x takes the output tiles
+  // x, x + 8, ..., every row tile of one before the next, so the row tiles
+  // that run together read each weight from their XCD's L2.
+  const int id = blockIdx.x + blockIdx.y * gridDim.x;
+  const bool by_xcd = gridDim.x % 8 == 0;
+  const int tile = by_xcd ? id / 8 / gridDim.y * 8 + id % 8 : blockIdx.x;
+  const int f0 = tile * T::kOutputs, b0 = (by_xcd ? id / 8 % gridDim.y : blockIdx.y) * T::kRows;
+  const int S = a.K / (8 * P);
   const uint64_t pos = a.ctl->position;
-
-  // Packed chunk of output f, step s, partial t: ((f / RW) S + s) 64 + (f % RW) P + t.
-  const u32x4* wsrc[kXgFeat];
-#pragma unroll
-  for (int j = 0; j < kXgFeat; ++j) {
-    const int f = f0 + j;
-    wsrc[j] = a.w + static_cast<uint64_t>(f / RW) * S * 64 + (f % RW) * P + t;
-  }
-  // Weights of a step: kXgFeat 16-byte chunks; two register sets alternate
-  // (a pass has an even number of steps), each loaded one step ahead.
-  u32x4 wa[kXgFeat], wb[kXgFeat];
-  auto load_w = [&](u32x4* w, int sg) {
-    const uint64_t at = static_cast<uint64_t>(sg < S ? sg : S - 1) * 64;  // past the end: reload the last step
-#pragma unroll
-    for (int j = 0; j < kXgFeat; ++j) w[j] = wsrc[j][at];
-  };
-  load_w(wa, 0);
-
-  // Piece q of row r of a pass: inputs 8q .. 8q + 7 of the pass (rows past
-  // B repeat row B - 1 and are never stored).
-  u32x4 xr[kPieces];
-  auto load_x = [&](int c) {
-#pragma unroll
-    for (int j = 0; j < kPieces; ++j) {
-      const int piece = threadIdx.x + j * kXgThreads, r = piece / (kXgChunk / 8), q = piece % (kXgChunk / 8);
-      const int b = min(b0 + r, a.B - 1);
-      xr[j] = *reinterpret_cast<const u32x4*>(a.x + static_cast<uint64_t>(b) * a.K + c * kXgChunk + 8 * q);
-    }
-  };
-  auto store_x = [&] {
-#pragma unroll
-    for (int j = 0; j < kPieces; ++j) {
-      const int piece = threadIdx.x + j * kXgThreads, r = piece / (kXgChunk / 8), q = piece % (kXgChunk / 8);
-      const float v[8] = {dl_bf16_lo(xr[j].x), dl_bf16_hi(xr[j].x), dl_bf16_lo(xr[j].y), dl_bf16_hi(xr[j].y),
-                          dl_bf16_lo(xr[j].z), dl_bf16_hi(xr[j].z), dl_bf16_lo(xr[j].w), dl_bf16_hi(xr[j].w)};
-      float* row = xs + r * row_floats;
-      if (a.permuted) {
-        // P-permuted: piece q holds chain elements 8 (q / P) .. + 7 of
-        // partial q % P (the pass starts on a block of 8 P inputs).
-        float4* dst = reinterpret_cast<float4*>(row + (q % P) * stride + 8 * (q / P));
-        dst[0] = make_float4(v[0], v[1], v[2], v[3]);
-        dst[1] = make_float4(v[4], v[5], v[6], v[7]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int i = 8 * q + e;
-          row[(i % P) * stride + i / P] = v[e];
-        }
-      }
-    }
-  };
-
-  float acc[kXgFeat * kXgPos];
-#pragma unroll
-  for (int i = 0; i < kXgFeat * kXgPos; ++i) acc[i] = 0.0f;
-  // One chain step (8 elements) of every (output, row) pair of the lane.
-  auto step = [&](const u32x4* w, int s) {
-    float wf[kXgFeat][8];
-#pragma unroll
-    for (int j = 0; j < kXgFeat; ++j) {
-      wf[j][0] = dl_bf16_lo(w[j].x); wf[j][1] = dl_bf16_hi(w[j].x);
-      wf[j][2] = dl_bf16_lo(w[j].y); wf[j][3] = dl_bf16_hi(w[j].y);
-      wf[j][4] = dl_bf16_lo(w[j].z); wf[j][5] = dl_bf16_hi(w[j].z);
-      wf[j][6] = dl_bf16_lo(w[j].w); wf[j][7] = dl_bf16_hi(w[j].w);
-    }
-#pragma unroll
-    for (int i = 0; i < kXgPos; ++i) {
-      const float* xp = xs + (pb + i) * row_floats + t * stride + 8 * s;
-      const float4 xa = *reinterpret_cast<const float4*>(xp);
-      const float4 xb = *reinterpret_cast<const float4*>(xp + 4);
-#pragma unroll
-      for (int j = 0; j < kXgFeat; ++j) {
-        float v = acc[j * kXgPos + i];
-        v = fma_rn(xa.x, wf[j][0], v);
-        v = fma_rn(xa.y, wf[j][1], v);
-        v = fma_rn(xa.z, wf[j][2], v);
-        v = fma_rn(xa.w, wf[j][3], v);
-        v = fma_rn(xb.x, wf[j][4], v);
-        v = fma_rn(xb.y, wf[j][5], v);
-        v = fma_rn(xb.z, wf[j][6], v);
-        v = fma_rn(xb.w, wf[j][7], v);
-        acc[j * kXgPos + i] = v;
-      }
-    }
-  };
-  static_assert(steps % 2 == 0, "the weight register sets alternate within a pass");
-  load_x(0);
-  for (int c = 0; c < passes; ++c) {
-    __syncthreads();  // every wavefront is done with the previous pass
-    store_x();
-    if (c + 1 < passes) load_x(c + 1);
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < steps; s += 2) {
-      const int sg = c * steps + s;
-      load_w(wb, sg + 1);
-      step(wa, s);
-      load_w(wa, sg + 2);
-      step(wb, s + 1);
-    }
-  }
-  chain_merge<P, kXgFeat * kXgPos>(acc);
-  if (t != 0) return;
-
   bool steer = false, capture = false;
-  uint32_t steer_mask = 0;
   if constexpr (EPI == kXgResidual) {
-    steer = a.res.steer != nullptr && a.res.layer == a.ctl->steer_layer;
+    steer = a.res.steer != nullptr && a.res.layer == a.ctl->steer_layer &&
+            ((a.ctl->steer_mask >> a.res.sequence) & 1u);
     capture = a.res.capture != nullptr && a.res.layer == a.ctl->capture_layer;
-    steer_mask = a.ctl->steer_mask;
   }
+  exact::tile_sums<T>(
+      S, 1024, 16 * P,
+      // Packed chunk of output f, step s, partial t: ((f / RW) S + s) 64 + (f % RW) P + t.
+      [&](int row, int piece) {
+        const int f = f0 + row;
+        return a.w + static_cast<uint64_t>(f / RW) * S * 64 + (f % RW) * P + piece;
+      },
+      // Rows past B repeat row B - 1 and are never stored.
+      [&](int row, int piece) {
+        return reinterpret_cast<const u32x4*>(a.x + static_cast<uint64_t>(min(b0 + row, a.B - 1)) * a.K) + piece;
+      },
+      [&](int output, int row, exact::f32x4 sum) {
+        const int b = b0 + row, f = f0 + output;
+        if (b >= a.B) return;
+        if constexpr (EPI == kXgGateUp) {
+          // [g 2j, g 2j+1, u 2j, u 2j+1], j = f / 4.
 #pragma unroll
-  for (int i = 0; i < kXgPos; ++i) {
-    const int b = b0 + pb + i;
-    if (b >= a.B) break;
-    if constexpr (EPI == kXgGateUp) {
-      // One P = 16 tile: [g 2j, g 2j+1, u 2j, u 2j+1], j = f0 / 4.
+          for (int o = 0; o < 2; ++o)
+            a.out[static_cast<uint64_t>(b) * (a.N / 2) + prefill::permuted(static_cast<uint32_t>(f / 2 + o), 32)] =
+                bf16_bits(silu_times(rbf(sum[o]), rbf(sum[2 + o])));
+        } else if constexpr (EPI == kXgResidual) {
+          // residual_store for four consecutive outputs of one sequence's row.
+          u32x2* h = reinterpret_cast<u32x2*>(a.res.h + static_cast<uint64_t>(b) * a.N + f);
+          const u32x2 old = *h;
+          const float was[4] = {dl_bf16_lo(old.x), dl_bf16_hi(old.x), dl_bf16_lo(old.y), dl_bf16_hi(old.y)};
+          float value[4];
 #pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        const uint32_t n = static_cast<uint32_t>(f0 / 2 + o);
-        a.out[static_cast<uint64_t>(b) * (a.N / 2) + prefill::permuted(n, 32)] =
-            bf16_bits(silu_times(rbf(acc[o * kXgPos + i]), rbf(acc[(2 + o) * kXgPos + i])));
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < kXgFeat; ++j) {
-        const int f = f0 + j;
-        const float y = acc[j * kXgPos + i];
-        if constexpr (EPI == kXgQ) {
-          a.out[static_cast<uint64_t>(b) * a.N + f] = bf16_bits(y);
-        } else if constexpr (EPI == kXgKV) {
-          if (f < a.kw)
-            a.out[static_cast<uint64_t>(b) * a.kw + f] = bf16_bits(y);
-          else
-            a.v_cache[static_cast<uint64_t>(b) * a.v_stride + static_cast<uint64_t>(f - a.kw) * a.cap + pos] =
-                bf16_bits(y);
+          for (int i = 0; i < 4; ++i) {
+            value[i] = rbf(was[i] + rbf(sum[i]));
+            if (steer) value[i] = rbf(value[i] + a.res.steer[static_cast<uint64_t>(a.res.sequence) * a.N + f + i]);
+          }
+          const u32x2 now = pack4(value);
+          *h = now;
+          if (capture)
+            *reinterpret_cast<u32x2*>(a.res.capture +
+                                      (static_cast<uint64_t>(a.res.sequence) * a.res.cap + pos + b) * a.N + f) = now;
         } else {
-          residual_store(a.res, f, b, y, pos, steer, capture, steer_mask);
+          const float value[4] = {sum[0], sum[1], sum[2], sum[3]};
+          if (EPI == kXgQ || f < a.kw) {
+            *reinterpret_cast<u32x2*>(a.out + static_cast<uint64_t>(b) * (EPI == kXgQ ? a.N : a.kw) + f) = pack4(value);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              a.v_cache[static_cast<uint64_t>(b) * a.v_stride + static_cast<uint64_t>(f + i - a.kw) * a.cap + pos] =
+                  bf16_bits(value[i]);
+          }
         }
-      }
-    }
-  }
+      });
 }
 
 // ------------------------------------------------------------------ LM head
@@ -3658,11 +3552,6 @@ void prepare_kernels_all(dl_plan* p) {
   const int D = c.hidden, QW = c.q_heads * c.head_dim, F = c.ffn;
   allow_lds(k_attn_pv, kPvLds);
   allow_lds(k_attn_pv_block, kPbLds);
-  allow_lds(k_xgemm<16, kXgQ>, xgemm_lds(16));
-  allow_lds(k_xgemm<32, kXgKV>, xgemm_lds(32));
-  allow_lds(k_xgemm<16, kXgResidual>, xgemm_lds(16));
-  allow_lds(k_xgemm<32, kXgResidual>, xgemm_lds(32));
-  allow_lds(k_xgemm<16, kXgGateUp>, xgemm_lds(16));
   allow_lds(k_qkv<1>, qkv_lds(1, D));
   allow_lds(k_qkv<2>, qkv_lds(2, D));
   allow_lds(k_qkv<4>, qkv_lds(4, D));
@@ -3743,13 +3632,20 @@ template <int G>
 void launch_head(dl_plan* p, hipStream_t s, const dl::HeadArgs& a) {
   dl::k_lm_head<G><<<p->head_blocks, dl::gemv_waves(G) * 64, p16_lds(G, a.D), s>>>(a);
 }
-// The many-row exact GEMM: grid (output blocks, row blocks).
+// The many-row exact GEMM: grid (output tiles, row tiles).  Each tile shape
+// leaves two workgroups per compute unit (80 and 64 KiB of LDS, 64
+// accumulators per lane), whose barriers do not fall together.  Measured for
+// 512 / 127 rows against tiles of twice the accumulators, one workgroup per
+// compute unit: gate/up 863 / 240 us against 901 / 239, O 149 / 45 against
+// 152 / 75, down 454 / 123 against 449 / 120, K/V 82 / 25 against 83 / 42
+// (the last two with two and three stage buffers: 454 against 474 us).
 template <int P, int EPI>
 void launch_xgemm(hipStream_t s, const dl::XgemmArgs& a) {
-  constexpr int tile_outputs = dl::kXgWN * (64 / P) * dl::kXgFeat;
-  require(a.N % tile_outputs == 0 && a.K % dl::kXgChunk == 0 && a.B > 0, "exact GEMM shape");
-  const dim3 grid(a.N / tile_outputs, (a.B + dl::kXgRows - 1) / dl::kXgRows);
-  dl::k_xgemm<P, EPI><<<grid, dl::kXgThreads, dl::xgemm_lds(P), s>>>(a);
+  using namespace dl::exact;
+  using T = std::conditional_t<P == 16, Tile<16, 4, 2, 1, 3, Order::kPermuted>, Tile<32, 8, 1, 1, 2, Order::kPermuted>>;
+  require(a.N % T::kOutputs == 0 && a.K % T::kInputs == 0 && a.B > 0, "exact GEMM shape");
+  const dim3 grid(a.N / T::kOutputs, (a.B + T::kRows - 1) / T::kRows);
+  dl::k_xgemm<T, EPI><<<grid, kThreads, 0, s>>>(a);
 }
 
 // The rows one step works on.  For the token loop they are the plan's
@@ -3775,14 +3671,13 @@ StepRows plan_rows(const dl_plan* p) {
 }
 
 // Whether step rows `r` run their projections through the many-row exact
-// GEMM (its shapes: widths that are whole passes of staged inputs).
+// GEMM (its shapes: widths that are whole stages of 8 P inputs).
 bool use_xgemm(const dl_plan* p, const StepRows& r) {
   const auto& c = p->model->cfg;
   const dl_qwen3* m = p->model;
   return r.rows >= static_cast<uint32_t>(dl::kXgMinRows) && r.x16 != nullptr && r.x32 != nullptr &&
          m->p_q == 16 && m->p_kv == 32 && m->p_o == 16 && m->p_gu == 16 && m->p_down == 32 &&
-         c.hidden % dl::kXgChunk == 0 && (uint64_t(c.q_heads) * c.head_dim) % dl::kXgChunk == 0 &&
-         c.ffn % dl::kXgChunk == 0;
+         c.hidden % 256 == 0 && (uint64_t(c.q_heads) * c.head_dim) % 128 == 0 && c.ffn % 256 == 0;
 }
 
 // Launches one decode-step kernel `which` of layer `l` with control `ctl`
@@ -3796,20 +3691,20 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
   const float scale = static_cast<float>(1.0 / std::sqrt(static_cast<double>(c.head_dim)));
   uint16_t* kc = p->k_cache + uint64_t(l) * p->cache_layer_stride + r.cache_base;
   uint16_t* vc = p->v_cache + uint64_t(l) * p->cache_layer_stride + r.cache_base;
+  const bool xg = use_xgemm(p, r);
   AttnArgs aa{ctl, r.q_raw, r.k_raw, m->q_norm[l], m->k_norm[l], p->rope, kc, vc, r.attn_seq_stride,
               r.scores, r.probs, r.att, static_cast<int>(c.q_heads), static_cast<int>(c.kv_heads),
-              static_cast<int>(p->cap), c.rms_eps, scale, r.pos_step};
-  const bool xg = use_xgemm(p, r);
+              static_cast<int>(p->cap), c.rms_eps, scale, r.pos_step, xg ? 1 : 0};
   switch (which) {
     case 0:
       if (xg) {
         prefill::launch_norm(s, prefill::NormArgs{r.h, m->input_norm[l], r.x16, r.x32, static_cast<int>(B), D,
                                                   c.rms_eps});
-        XgemmArgs qa{ctl, r.x16, reinterpret_cast<const u32x4*>(m->qkv[l]), static_cast<int>(B), QW, D, 1,
+        XgemmArgs qa{ctl, r.x16, reinterpret_cast<const u32x4*>(m->qkv[l]), static_cast<int>(B), QW, D,
                      r.q_raw, nullptr, 0, KW, static_cast<int>(p->cap), {}};
         launch_xgemm<16, kXgQ>(s, qa);
         XgemmArgs kva{ctl, r.x32, reinterpret_cast<const u32x4*>(m->qkv[l] + uint64_t(QW) * D),
-                      static_cast<int>(B), 2 * KW, D, 1, r.k_raw, vc, r.v_append_stride, KW,
+                      static_cast<int>(B), 2 * KW, D, r.k_raw, vc, r.v_append_stride, KW,
                       static_cast<int>(p->cap), {}};
         launch_xgemm<32, kXgKV>(s, kva);
         break;
@@ -3895,7 +3790,7 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
         ResidualArgs oa{ctl, r.att, reinterpret_cast<const u32x4*>(m->o[l]), r.h, nullptr, nullptr, QW, D,
                         static_cast<int>(p->cap), static_cast<int>(l), 0, r.same_sequence, r.sequence};
         launch_xgemm<16, kXgResidual>(
-            s, XgemmArgs{ctl, r.att, oa.w, static_cast<int>(B), D, QW, 0, nullptr, nullptr, 0, 0, 0, oa});
+            s, XgemmArgs{ctl, r.att, oa.w, static_cast<int>(B), D, QW, nullptr, nullptr, 0, 0, 0, oa});
         break;
       }
       for_row_groups(B, kWideRows, [&](uint32_t r0, int g, int rows) {
@@ -3914,7 +3809,7 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
                                                   c.rms_eps});
         // SiLU(g) * u rows go to act in P32 order, the order the down GEMM stages.
         launch_xgemm<16, kXgGateUp>(s, XgemmArgs{ctl, r.x16, reinterpret_cast<const u32x4*>(m->gu[l]),
-                                                 static_cast<int>(B), 2 * F, D, 1, r.act, nullptr, 0, 0, 0, {}});
+                                                 static_cast<int>(B), 2 * F, D, r.act, nullptr, 0, 0, 0, {}});
         break;
       }
       for_row_groups(B, kWideRows, [&](uint32_t r0, int g, int rows) {
@@ -3931,7 +3826,7 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
         ResidualArgs da{ctl, r.act, reinterpret_cast<const u32x4*>(m->down[l]), r.h, p->capture, p->steer, F, D,
                         static_cast<int>(p->cap), static_cast<int>(l), 0, r.same_sequence, r.sequence};
         launch_xgemm<32, kXgResidual>(
-            s, XgemmArgs{ctl, r.act, da.w, static_cast<int>(B), D, F, 1, nullptr, nullptr, 0, 0, 0, da});
+            s, XgemmArgs{ctl, r.act, da.w, static_cast<int>(B), D, F, nullptr, nullptr, 0, 0, 0, da});
         break;
       }
       // Staging in blocks needs whole blocks of inputs; other widths keep

@@ -76,6 +76,15 @@ def test_exact_prefill_equals_token_loop(model2, length):
     assert_same(model2, a, b, length + 6)
 
 
+@pytest.mark.parametrize("rows", [16, 31, 32, 33, 63, 65, 97])
+def test_exact_prefill_row_tiles(model1, rows):
+    """Chunks around the many-row GEMM's 32-row tiles: its first row count, a
+    whole tile, one row less and more, and several tiles with a remainder."""
+    prompt = [int(t) for t in np.random.default_rng(rows).integers(0, 2048, rows + 1)]
+    a, b = run_pair(model1, prompt, 2, capacity=128)
+    assert_same(model1, a, b, rows + 3)
+
+
 def test_exact_prefill_across_the_fused_attention_limit(model1):
     """A 1600-id prompt: chunks below 1536 keys use the one-kernel attention,
     the later ones the split long-context kernels."""
