@@ -29,34 +29,36 @@
 namespace dl::exact {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 typedef __attribute__((address_space(3))) void lds_ptr;
 typedef __attribute__((address_space(1))) void global_ptr;
 
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * 64;
-
 enum class Order { kPermuted, kNatural };
 
-// A workgroup of 8 wavefronts computes TM x TN tiles of 32 outputs x 32 rows;
-// Split wavefronts share a tile, each with P / Split of its chains (16 P /
-// Split accumulators per lane).  Block b of instruction w of wavefront c holds
-// chain t = (P / 2) b + Split w + c, so offsets P/2 .. Split merge inside a
-// lane and only the last log2(Split) offsets cross wavefronts.
-template <int P_, int Split_, int TM_, int TN_, int Ring_, Order Weights_>
+// A workgroup computes TM x TN tiles of Edge outputs x Edge rows (32, or 16
+// with the four-block v_mfma_f32_16x16x1_4b_f32 where there are few rows);
+// Split wavefronts share a tile, each with P / Split of its chains.  Block b
+// of instruction w of wavefront c holds chain t = (P / Blocks) b + Split w + c,
+// so the offsets P/2 .. Split merge inside a lane and only the last
+// log2(Split) offsets cross wavefronts.  A stage is Groups x 8 chain steps.
+template <int P_, int Edge_, int Split_, int TM_, int TN_, int Groups_, int Ring_, Order Weights_, Order Rows_>
 struct Tile {
-  static constexpr int P = P_, Split = Split_, TM = TM_, TN = TN_, kRing = Ring_;
-  static constexpr Order kWeights = Weights_;
-  static constexpr int W = P / Split / 2;  // instructions per chain step
-  static constexpr int kOutputs = 32 * TM, kRows = 32 * TN;
+  static constexpr int P = P_, Edge = Edge_, Split = Split_, TM = TM_, TN = TN_, kGroups = Groups_, kRing = Ring_;
+  static constexpr Order kWeights = Weights_, kRowOrder = Rows_;
+  static constexpr int kBlocks = 64 / Edge, kChains = P / kBlocks;  // chains per block
+  static constexpr int W = kChains / Split;                         // instructions per chain step
+  static constexpr int kWaves = TM * TN * Split, kThreads = 64 * kWaves;
+  static constexpr int kOutputs = Edge * TM, kRows = Edge * TN;
   static constexpr int kStageRows = kOutputs + kRows;
-  static constexpr int kRowBytes = 16 * P;  // 8 P inputs in BF16
-  static constexpr int kInputs = 8 * P;     // inputs per stage
-  static constexpr int kLoads = kStageRows * P / 64 / kWaves;  // 1 KiB loads per wavefront and stage
+  static constexpr int kPieces = kGroups * P, kRowBytes = 16 * kPieces;  // per stage row
+  static constexpr int kInputs = 8 * kPieces;                            // inputs per stage
+  static constexpr int kLoads = kStageRows * kPieces / 64 / kWaves;      // 1 KiB loads per wavefront and stage
   static constexpr int kStageBytes = kStageRows * kRowBytes;
-  static_assert(TM * TN * Split == kWaves && (P == 16 || P == 32), "eight wavefronts, 16 or 32 partials");
-  static_assert(W == 2 || W == 4, "64 or 128 accumulators per lane");
-  static_assert(kRing == 2 || kRing == 3, "two or three stage buffers");
+  static constexpr int kRegs = 1024 / 64 * (Edge == 32 ? 2 : 1);  // accumulators per instruction
+  static_assert((Edge == 32 || Edge == 16) && (P == 16 || P == 32) && W >= 1 && kChains % Split == 0, "tile shape");
+  static_assert(kStageRows * kPieces % (64 * kWaves) == 0, "whole loads per wavefront");
+  static_assert(kRing >= 2 && kRing <= 4, "two to four stage buffers");
 };
 
 // s_waitcnt immediates: at most n vector-memory operations outstanding (vmcnt
@@ -65,20 +67,20 @@ struct Tile {
 constexpr unsigned vm_wait(unsigned n) { return 0x0f70u | (n & 0xfu) | ((n >> 4) << 14); }
 constexpr unsigned vm_lds_wait(unsigned n) { return 0x0070u | (n & 0xfu) | ((n >> 4) << 14); }
 
-// A lane's operands of one 32-row tile for half a stage (chain steps 4 half ..
-// + 3): block b = lane / 32, row lane % 32.
+// A lane's operands of one tile for half a group (chain steps 4 half .. + 3):
+// block b = lane / Edge, row lane % Edge.
 template <class T, Order O>
 struct Operands;
 
 template <class T>
 struct Operands<T, Order::kPermuted> {
-  u32x2 v[T::W];  // four steps of chain (P / 2) b + Split w + c
+  u32x2 v[T::W];  // four steps of chain kChains b + Split w + c
   __device__ __forceinline__ void load(const uint8_t* stage, int first_row, int half, int lane, int c) {
-    const int b = lane / 32, r = lane % 32;
-    const uint8_t* row = stage + (first_row + r) * T::kRowBytes + half * 8;
+    const int b = lane / T::Edge, r = lane % T::Edge;
+    const uint8_t* row = stage + (first_row + r) * T::kRowBytes + half / 2 * T::P * 16 + half % 2 * 8;
 #pragma unroll
     for (int w = 0; w < T::W; ++w)
-      v[w] = *reinterpret_cast<const u32x2*>(row + ((T::P / 2 * b + T::Split * w + c) ^ (r % 16)) * 16);
+      v[w] = *reinterpret_cast<const u32x2*>(row + ((T::kChains * b + T::Split * w + c) ^ (r % 16)) * 16);
   }
   __device__ __forceinline__ float at(int w, int e, uint32_t) const {
     const uint32_t word = e < 2 ? v[w].x : v[w].y;
@@ -90,23 +92,14 @@ template <class T>
 struct Operands<T, Order::kNatural> {
   uint32_t v[4][T::W];  // per step, the word that holds the input (half c % 2 of it)
   __device__ __forceinline__ void load(const uint8_t* stage, int first_row, int half, int lane, int c) {
-    const int b = lane / 32, r = lane % 32;
+    const int b = lane / T::Edge, r = lane % T::Edge;
     const uint8_t* row = stage + (first_row + r) * T::kRowBytes;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int base = T::P * (4 * half + e) + T::P / 2 * b;  // a multiple of 8
-      if constexpr (T::Split == 2) {
-        const u32x4 q = *reinterpret_cast<const u32x4*>(row + ((base / 8) ^ (r % 16)) * 16);
-        v[e][0] = q.x;
-        v[e][1] = q.y;
-        v[e][2] = q.z;
-        v[e][3] = q.w;
-      } else {
 #pragma unroll
-        for (int w = 0; w < T::W; ++w) {
-          const int input = base + T::Split * w;
-          v[e][w] = *reinterpret_cast<const uint32_t*>(row + ((input / 8) ^ (r % 16)) * 16 + (input % 8) * 2 + c / 2 * 4);
-        }
+      for (int w = 0; w < T::W; ++w) {
+        const int input = T::P * (4 * half + e) + T::kChains * b + T::Split * w;
+        v[e][w] = *reinterpret_cast<const uint32_t*>(row + ((input / 8) ^ (r % 16)) * 16 + (input % 8 + c / 2 * 2) * 2);
       }
     }
   }
@@ -116,18 +109,35 @@ struct Operands<T, Order::kNatural> {
   }
 };
 
+template <int Edge>
+struct Products;
+template <>
+struct Products<32> {
+  typedef f32x32 Sum;
+  static __device__ __forceinline__ Sum step(float a, float b, Sum c) {
+    return __builtin_amdgcn_mfma_f32_32x32x1f32(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct Products<16> {
+  typedef f32x16 Sum;
+  static __device__ __forceinline__ Sum step(float a, float b, Sum c) {
+    return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
+  }
+};
+
 // The sums of one workgroup tile over `stages` stages.  a_src(row, piece) and
-// b_src(row, piece) give the address of a 16-byte piece of output row / input
-// row of the tile in the first stage; the same piece of the next stage lies
-// a_step / b_step bytes further.  Each piece lands in LDS at piece ^ (row % 16)
-// of its row, so an operand read spreads over the banks while the loads of 4
-// lanes stay 64 contiguous bytes.
+// b_src(row, piece) give the address of 16-byte piece `piece` (below P) of
+// output row / input row of the tile in the first group of 8 steps; the same
+// piece of the next group lies a_step / b_step bytes further.  Each piece
+// lands in LDS at piece ^ (row % 16) of its row, so an operand read spreads
+// over the banks while the loads of 4 lanes stay 64 contiguous bytes.
 //
-// Stages pass through a ring of three LDS buffers by direct global-to-LDS
-// loads.  Half way through a stage, one barrier finds the next stage in LDS
+// Stages pass through a ring of LDS buffers by direct global-to-LDS loads.
+// Ahead of a stage's last half group, one barrier finds the next stage in LDS
 // and every wavefront past its reads of this one, whose buffer the stage
-// after the next two then takes; the operands of each half are read while the
-// half before is multiplied.  Loads past the last stage repeat it so that
+// kRing later then takes; the operands of each half group are read while the
+// one before is multiplied.  Loads past the last stage repeat it so that
 // every wait counts the same loads.  The buffers are separate LDS objects: the
 // compiler then adds no waits of its own between the loads in flight and the
 // operand reads.
@@ -137,104 +147,112 @@ struct Operands<T, Order::kNatural> {
 template <class T, class ASrc, class BSrc, class Finish>
 __device__ __forceinline__ void tile_sums(int stages, uint32_t a_step, uint32_t b_step, ASrc&& a_src, BSrc&& b_src,
                                           Finish&& finish) {
-  constexpr int kExchange = kWaves * 4 * 64 * sizeof(f32x4);
+  constexpr int kTileGroups = T::Edge == 32 ? 4 : 1;  // groups of four outputs per lane
+  constexpr int kExchange = T::Split > 1 ? T::kWaves * kTileGroups * 64 * sizeof(f32x4) : 16;
   __shared__ __align__(1024) uint8_t s0[T::kStageBytes > kExchange ? T::kStageBytes : kExchange], s1[T::kStageBytes],
-      s2[T::kRing == 3 ? T::kStageBytes : 16];
+      s2[T::kRing > 2 ? T::kStageBytes : 16], s3[T::kRing > 3 ? T::kStageBytes : 16];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int c = wave % T::Split, tile = wave / T::Split;
-  const int a_row = 32 * (tile / T::TN), b_row = 32 * (tile % T::TN);
+  const int a_row = T::Edge * (tile / T::TN), b_row = T::Edge * (tile % T::TN);
   const uint32_t select = c % 2 ? 0x03020c0cu : 0x01000c0cu;
 
   const uint8_t* src[T::kLoads];
   uint32_t step[T::kLoads];
 #pragma unroll
   for (int j = 0; j < T::kLoads; ++j) {
-    const int slot = (kWaves * j + wave) * 64 + lane;
-    const int row = slot / T::P, piece = (slot % T::P) ^ (row % 16);
+    const int slot = (T::kWaves * j + wave) * 64 + lane;
+    const int row = slot / T::kPieces, piece = (slot % T::kPieces) ^ (row % 16);
     // A 1 KiB unit lies wholly in the weights or in the rows.
-    const bool weights = (kWaves * j + wave) * 64 / T::P < T::kOutputs;
-    src[j] = reinterpret_cast<const uint8_t*>(weights ? a_src(row, piece) : b_src(row - T::kOutputs, piece));
-    step[j] = weights ? a_step : b_step;
+    const bool weights = (T::kWaves * j + wave) * 64 / T::kPieces < T::kOutputs;
+    const uint32_t group = weights ? a_step : b_step;
+    src[j] = reinterpret_cast<const uint8_t*>(weights ? a_src(row, piece % T::P) : b_src(row - T::kOutputs, piece % T::P)) +
+             piece / T::P * group;
+    step[j] = T::kGroups * group;
   }
   auto issue = [&](int s, uint8_t* buffer) {
 #pragma unroll
     for (int j = 0; j < T::kLoads; ++j)
       __builtin_amdgcn_global_load_lds((const global_ptr*)(src[j] + static_cast<uint64_t>(s) * step[j]),
-                                       (lds_ptr*)(buffer + (kWaves * j + wave) * 1024), 16, 0, 0);
+                                       (lds_ptr*)(buffer + (T::kWaves * j + wave) * 1024), 16, 0, 0);
   };
 
-  f32x32 acc[T::W];
+  typename Products<T::Edge>::Sum acc[T::W];
 #pragma unroll
   for (int w = 0; w < T::W; ++w)
 #pragma unroll
-    for (int r = 0; r < 32; ++r) acc[w][r] = 0.0f;
+    for (int r = 0; r < T::kRegs; ++r) acc[w][r] = 0.0f;
 
   struct Half {
     Operands<T, T::kWeights> a;
-    Operands<T, Order::kPermuted> b;
+    Operands<T, T::kRowOrder> b;
+  } f[2];
+  auto load_half = [&](const uint8_t* buffer, int half) {
+    f[half % 2].a.load(buffer, a_row, half, lane, c);
+    f[half % 2].b.load(buffer, T::kOutputs + b_row, half, lane, c);
   };
-  auto load_half = [&](const uint8_t* buffer, int half, Half& f) {
-    f.a.load(buffer, a_row, half, lane, c);
-    f.b.load(buffer, T::kOutputs + b_row, half, lane, c);
-  };
-  auto multiply = [&](const Half& f) {
+  auto multiply = [&](int half) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int w = 0; w < T::W; ++w)
-        acc[w] = __builtin_amdgcn_mfma_f32_32x32x1f32(f.a.at(w, e, select), f.b.at(w, e, 0), acc[w], 0, 0, 0);
+        acc[w] = Products<T::Edge>::step(f[half % 2].a.at(w, e, select), f[half % 2].b.at(w, e, select), acc[w]);
   };
 
   constexpr int kAhead = (T::kRing - 2) * T::kLoads;  // loads in flight past the next stage's
   issue(0, s0);
   issue(min(1, stages - 1), s1);
-  if constexpr (T::kRing == 3) issue(min(2, stages - 1), s2);
+  if constexpr (T::kRing > 2) issue(min(2, stages - 1), s2);
+  if constexpr (T::kRing > 3) issue(min(3, stages - 1), s3);
   __builtin_amdgcn_s_waitcnt(vm_wait(kAhead + T::kLoads));
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
-  Half f0, f1;
-  load_half(s0, 0, f0);
+  load_half(s0, 0);
   int s = 0;
   auto one = [&](uint8_t* current, const uint8_t* next) {
-    load_half(current, 1, f1);
-    multiply(f0);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(vm_lds_wait(kAhead));
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    load_half(next, 0, f0);
-    issue(min(s + T::kRing, stages - 1), current);
-    multiply(f1);
+#pragma unroll
+    for (int half = 0; half < 2 * T::kGroups; ++half) {
+      if (half + 1 < 2 * T::kGroups) {
+        load_half(current, half + 1);
+      } else {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(vm_lds_wait(kAhead));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        load_half(next, 0);
+        issue(min(s + T::kRing, stages - 1), current);
+      }
+      multiply(half);
+    }
     __builtin_amdgcn_sched_barrier(0);
     ++s;
   };
-  if constexpr (T::kRing == 3) {
-    while (s + 3 <= stages) {
-      one(s0, s1);
-      one(s1, s2);
-      one(s2, s0);
-    }
-    if (s < stages) one(s0, s1);
-    if (s < stages) one(s1, s2);
-  } else {
-    while (s + 2 <= stages) {
-      one(s0, s1);
-      one(s1, s0);
-    }
-    if (s < stages) one(s0, s1);
+  while (s + T::kRing <= stages) {
+    one(s0, s1);
+    one(s1, T::kRing > 2 ? s2 : s0);
+    if constexpr (T::kRing > 2) one(s2, T::kRing > 3 ? s3 : s0);
+    if constexpr (T::kRing > 3) one(s3, s0);
   }
+  if (s < stages) one(s0, s1);
+  if (T::kRing > 2 && s < stages) one(s1, s2);
+  if (T::kRing > 3 && s < stages) one(s2, s3);
   __builtin_amdgcn_s_waitcnt(vm_lds_wait(0));  // no load outlives the ring
 
-  // Register r of a block: row lane % 32, output 8 (r / 4) + 4 (lane / 32) +
-  // r % 4.  Offset P/2 merges the blocks, the next ones instructions.
-  f32x4 part[4];
+  // Registers of a block: row lane % Edge, outputs 4 (lane / Edge) + i (and
+  // + 8 g of a 32-wide tile).  The offsets from P / 2 down to kChains merge
+  // the blocks, the next ones instructions.
+  f32x4 part[kTileGroups];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
+  for (int g = 0; g < kTileGroups; ++g) {
     f32x4 sum[T::W];
 #pragma unroll
     for (int w = 0; w < T::W; ++w)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sum[w][i] = acc[w][4 * g + i] + acc[w][16 + 4 * g + i];
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (T::Edge == 32)
+          sum[w][i] = acc[w][4 * g + i] + acc[w][16 + 4 * g + i];
+        else
+          sum[w][i] = (acc[w][i] + acc[w][8 + i]) + (acc[w][4 + i] + acc[w][12 + i]);
+      }
 #pragma unroll
     for (int off = T::W / 2; off; off /= 2)
 #pragma unroll
@@ -243,29 +261,35 @@ __device__ __forceinline__ void tile_sums(int stages, uint32_t a_step, uint32_t 
         for (int i = 0; i < 4; ++i) sum[w][i] = sum[w][i] + sum[w + off][i];
     part[g] = sum[0];
   }
-  // The remaining offsets across the tile's wavefronts through LDS: wavefront
-  // c finishes the output groups [4 c / Split, 4 (c + 1) / Split); with eight
-  // wavefronts per tile, the halves (lane / 32) of group c / 2.
+  if constexpr (T::Split == 1) {
+#pragma unroll
+    for (int g = 0; g < kTileGroups; ++g) finish(a_row + 8 * g + 4 * (lane / T::Edge), b_row + lane % T::Edge, part[g]);
+    return;
+  }
+  // The remaining offsets across the tile's wavefronts through LDS.
+  // Wavefront c finishes its share of the tile: whole groups while there are
+  // enough, else a share of the lanes of one group.
   f32x4* exchange = reinterpret_cast<f32x4*>(s0);  // [tile][c][group][lane]
   __builtin_amdgcn_s_barrier();
 #pragma unroll
-  for (int g = 0; g < 4; ++g) exchange[((tile * T::Split + c) * 4 + g) * 64 + lane] = part[g];
+  for (int g = 0; g < kTileGroups; ++g) exchange[((tile * T::Split + c) * kTileGroups + g) * 64 + lane] = part[g];
   __syncthreads();
-  constexpr int kGroups = T::Split >= 4 ? 1 : 4 / T::Split;
+  constexpr int kShare = kTileGroups >= T::Split ? kTileGroups / T::Split : 1;  // groups per wavefront
+  constexpr int kLanes = kTileGroups >= T::Split ? 1 : T::Split / kTileGroups;  // wavefronts per group
 #pragma unroll
-  for (int i = 0; i < kGroups; ++i) {
-    const int g = T::Split == 8 ? c / 2 : c * kGroups + i;
-    if (T::Split == 8 && lane / 32 != c % 2) continue;
+  for (int i = 0; i < kShare; ++i) {
+    const int g = kLanes > 1 ? c / kLanes : c * kShare + i;
+    if (kLanes > 1 && lane / (64 / kLanes) != c % kLanes) continue;
     f32x4 sum[T::Split];
 #pragma unroll
-    for (int k = 0; k < T::Split; ++k) sum[k] = exchange[((tile * T::Split + k) * 4 + g) * 64 + lane];
+    for (int k = 0; k < T::Split; ++k) sum[k] = exchange[((tile * T::Split + k) * kTileGroups + g) * 64 + lane];
 #pragma unroll
     for (int off = T::Split / 2; off; off /= 2)
 #pragma unroll
       for (int k = 0; k < off; ++k)
 #pragma unroll
         for (int j = 0; j < 4; ++j) sum[k][j] = sum[k][j] + sum[k + off][j];
-    finish(a_row + 8 * g + 4 * (lane / 32), b_row + lane % 32, sum[0]);
+    finish(a_row + 8 * g + 4 * (lane / T::Edge), b_row + lane % T::Edge, sum[0]);
   }
 }
 

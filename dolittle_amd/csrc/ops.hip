@@ -14,9 +14,12 @@
 //    CPU oracle); sqrt and division are IEEE correctly rounded.
 #include <algorithm>
 #include <cstdint>
+#include <utility>
+#include <type_traits>
 
 #include "dl_device.h"
 #include "dl_internal.h"
+#include "exact_mfma.h"
 
 namespace dl {
 namespace {
@@ -71,6 +74,234 @@ __global__ __launch_bounds__(kThreads) void projection_rowmajor(const T* __restr
   }
 }
 
+// The same chains on the FP32 matrix cores (exact_mfma.h), row-major BF16
+// operands in natural order: whole stages of inputs, 16-byte aligned rows.
+// Rows and outputs past the end repeat the last one and are not stored.  Few
+// rows are bound by the weight stream (16 rows of 4096 x 12288: 31 us, 3.2
+// TB/s; 384 us with one lane per partial reading 2 bytes at a time), many by
+// the FP32 MFMA rate and the operand widening.
+template <class T>
+__global__ __launch_bounds__(T::kThreads) __attribute__((amdgpu_waves_per_eu(T::Edge == 32 ? 4 : T::P / 8))) void k_project_tiles(const uint16_t* __restrict__ x,
+                                                               const uint16_t* __restrict__ w,
+                                                               uint16_t* __restrict__ y, uint64_t rows, uint64_t in_w,
+                                                               uint64_t out_w, const uint64_t* out_pos) {
+  const uint64_t id = blockIdx.x + static_cast<uint64_t>(blockIdx.y) * gridDim.x;
+  // XCD x takes the output tiles x, x + 8, ..., all row tiles of one together.
+  const bool by_xcd = gridDim.x % 8 == 0;
+  const uint64_t tile = by_xcd ? id / 8 / gridDim.y * 8 + id % 8 : blockIdx.x;
+  const uint64_t o0 = tile * T::kOutputs, r0 = (by_xcd ? id / 8 % gridDim.y : blockIdx.y) * T::kRows;
+  uint16_t* out = y + (out_pos ? *out_pos * out_w : 0);
+  const bool vector = out_w % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0;
+  exact::tile_sums<T>(
+      static_cast<int>(in_w / T::kInputs), 16 * T::P, 16 * T::P,
+      [&](int row, int piece) {
+        return reinterpret_cast<const u32x4*>(w + min(o0 + row, out_w - 1) * in_w) + piece;
+      },
+      [&](int row, int piece) {
+        return reinterpret_cast<const u32x4*>(x + min(r0 + row, rows - 1) * in_w) + piece;
+      },
+      [&](int output, int row, exact::f32x4 sum) {
+        const uint64_t r = r0 + row, o = o0 + output;
+        if (r >= rows || o >= out_w) return;
+        uint16_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = dl_f32_to_bf16(sum[i]);
+        uint16_t* at = out + r * out_w + o;
+        if (vector) {
+          *reinterpret_cast<u32x2*>(at) = u32x2{v[0] | (static_cast<uint32_t>(v[1]) << 16),
+                                                v[2] | (static_cast<uint32_t>(v[3]) << 16)};
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (o + i < out_w) at[i] = v[i];
+        }
+      });
+}
+
+// One row, bound by the weight stream.  A wavefront owns 8 outputs, 8 lanes
+// each: lane (r, j) holds the P / 8 chains (P / 8) j .. of output r, which are
+// neighbours in a row-major row, so one LDS read brings a step of all of them.
+// Its weights stream through its own ring of kRing LDS buffers (256 inputs of
+// 8 rows, 4 KiB) by direct global-to-LDS loads, so what is in flight takes no
+// registers and no wavefront waits for another; the input row is staged once
+// per workgroup as FP32.  Piece p of row r lies at p ^ (P / 8 r): the 8 rows of
+// a read fall in distinct banks.
+//
+// Measured (one lane per partial reading 2 bytes at a time / the matrix-core
+// tiles of 16 rows / this): 4096 x 4096 98 / 14.5 / 12.4 us, 4096 x 1024 59 /
+// 13 / 9.7, 4096 x 12288 166 / 31 / 22.3 (4.5 TB/s), 12288 x 4096 185 / 34 /
+// 29, 4096 x 151936 202 us (6.2 TB/s).
+template <int P_, int MaxInputs_>
+struct RowTile {
+  static constexpr int P = P_, kMaxInputs = MaxInputs_, kWaves = 2, kRing = 4;
+  static constexpr int kRows = 8, C = P / 8;  // outputs per wavefront, chains per lane
+  static constexpr int kInputs = 256, kRowBytes = 2 * kInputs, kPieces = kInputs / 8;
+  static constexpr int kStageBytes = kRows * kRowBytes, kLoads = kStageBytes / 1024;
+  static constexpr int kThreads = 64 * kWaves;
+};
+
+template <int... I, class F>
+__device__ __forceinline__ void for_each_index(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+// Stage buffer I of every wavefront: a separate LDS object per stage, so the
+// compiler adds no waits between the loads in flight and the reads.
+template <class T, int I>
+__device__ __forceinline__ uint8_t* row_stage(int wave) {
+  __shared__ __align__(1024) uint8_t stage[T::kWaves * T::kStageBytes];
+  return stage + wave * T::kStageBytes;
+}
+
+template <class T>
+__global__ __launch_bounds__(T::kThreads) void k_project_row(const uint16_t* __restrict__ x,
+                                                             const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
+                                                             uint64_t in_w, uint64_t out_w, const uint64_t* out_pos) {
+  constexpr int P = T::P, C = T::C;
+  // Static: reads of dynamic LDS would wait for every load in flight.
+  __shared__ __align__(16) float xs[T::kMaxInputs];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int r = lane / 8, j = lane % 8;
+  const uint64_t o0 = (static_cast<uint64_t>(blockIdx.x) * T::kWaves + wave) * T::kRows;
+  const int stages = static_cast<int>(in_w / T::kInputs), chunks = static_cast<int>(in_w / 8);
+
+  // The input comes before the weights: loads retire in order.
+  constexpr int kChunks = T::kMaxInputs / 8 / T::kThreads;
+  u32x4 xv[kChunks];
+#pragma unroll
+  for (int i = 0; i < kChunks; ++i)
+    xv[i] = reinterpret_cast<const u32x4*>(x)[min(static_cast<int>(threadIdx.x) + i * T::kThreads, chunks - 1)];
+  __builtin_amdgcn_sched_barrier(0);
+  const uint8_t* src[T::kLoads];
+#pragma unroll
+  for (int i = 0; i < T::kLoads; ++i) {
+    const int slot = i * 64 + lane, row = slot / T::kPieces, piece = (slot % T::kPieces) ^ (C * row % T::kPieces);
+    src[i] = reinterpret_cast<const uint8_t*>(w + min(o0 + row, out_w - 1) * in_w) + piece * 16;
+  }
+  auto issue = [&](int s, uint8_t* buffer) {
+#pragma unroll
+    for (int i = 0; i < T::kLoads; ++i)
+      __builtin_amdgcn_global_load_lds((const exact::global_ptr*)(src[i] + static_cast<uint64_t>(s) * T::kRowBytes),
+                                       (exact::lds_ptr*)(buffer + i * 1024), 16, 0, 0);
+  };
+  for_each_index(std::make_integer_sequence<int, T::kRing>{}, [&](auto i) {
+    issue(min(static_cast<int>(i.value), stages - 1), row_stage<T, i.value>(wave));
+  });
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < kChunks; ++i) {
+    const int chunk = threadIdx.x + i * T::kThreads;
+    if (chunk < chunks) {
+      float4* dst = reinterpret_cast<float4*>(xs + 8 * chunk);
+      dst[0] = make_float4(dl_bf16_lo(xv[i].x), dl_bf16_hi(xv[i].x), dl_bf16_lo(xv[i].y), dl_bf16_hi(xv[i].y));
+      dst[1] = make_float4(dl_bf16_lo(xv[i].z), dl_bf16_hi(xv[i].z), dl_bf16_lo(xv[i].w), dl_bf16_hi(xv[i].w));
+    }
+  }
+  __syncthreads();
+
+  float acc[C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) acc[i] = 0.0f;
+  auto one = [&](int s, uint8_t* buffer) {
+    __builtin_amdgcn_s_waitcnt(exact::vm_wait((T::kRing - 1) * T::kLoads));  // stage s has landed
+    __builtin_amdgcn_sched_barrier(0);
+    const uint8_t* row = buffer + r * T::kRowBytes;
+    const float* xt = xs + s * T::kInputs + C * j;
+    const int swizzle = C * r % T::kPieces;
+#pragma unroll
+    for (int e = 0; e < T::kInputs / P; ++e) {
+      const int input = P * e + C * j;
+      const uint8_t* at = row + ((input / 8) ^ swizzle) * 16 + (input % 8) * 2;
+      if constexpr (C == 2) {
+        const uint32_t v = *reinterpret_cast<const uint32_t*>(at);
+        const float2 xe = *reinterpret_cast<const float2*>(xt + P * e);
+        acc[0] = fma_rn(xe.x, dl_bf16_lo(v), acc[0]);
+        acc[1] = fma_rn(xe.y, dl_bf16_hi(v), acc[1]);
+      } else {
+        const u32x2 v = *reinterpret_cast<const u32x2*>(at);
+        const float4 xe = *reinterpret_cast<const float4*>(xt + P * e);
+        acc[0] = fma_rn(xe.x, dl_bf16_lo(v.x), acc[0]);
+        acc[1] = fma_rn(xe.y, dl_bf16_hi(v.x), acc[1]);
+        acc[2] = fma_rn(xe.z, dl_bf16_lo(v.y), acc[2]);
+        acc[3] = fma_rn(xe.w, dl_bf16_hi(v.y), acc[3]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // the buffer is read: stage s + kRing may take it
+    issue(min(s + T::kRing, stages - 1), buffer);
+  };
+  for (int s = 0; s < stages; s += T::kRing) {
+    for_each_index(std::make_integer_sequence<int, T::kRing>{}, [&](auto i) {
+      if (s + i.value < stages) one(s + i.value, row_stage<T, i.value>(wave));
+    });
+  }
+  __builtin_amdgcn_s_waitcnt(exact::vm_wait(0));  // no load outlives the wavefront
+
+  // Offsets P / 2 .. C across the output's lanes, the rest within the lane.
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    acc[i] = acc[i] + row_down<4>(acc[i]);
+    acc[i] = acc[i] + row_down<2>(acc[i]);
+    acc[i] = acc[i] + row_down<1>(acc[i]);
+  }
+#pragma unroll
+  for (int off = C / 2; off; off /= 2)
+#pragma unroll
+    for (int i = 0; i < off; ++i) acc[i] = acc[i] + acc[i + off];
+  if (j == 0 && o0 + r < out_w) y[(out_pos ? *out_pos * out_w : 0) + o0 + r] = dl_f32_to_bf16(acc[0]);
+}
+
+template <class T>
+void launch_project_row(hipStream_t s, const uint16_t* x, const uint16_t* w, uint16_t* y, uint64_t in_w,
+                        uint64_t out_w, const uint64_t* out_pos) {
+  k_project_row<T><<<static_cast<unsigned>(ceil_div(out_w, T::kRows * T::kWaves)), T::kThreads, 0, s>>>(
+      x, w, y, in_w, out_w, out_pos);
+}
+
+// Whether a BF16 projection runs on k_project_tiles: whole stages of 256
+// inputs and 16-byte aligned operands.
+bool tiled_projection(const void* x, const void* w, uint64_t in_w) {
+  return in_w % 256 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+}
+
+// Tiles of 16 rows up to kFewRows, of 32 above: the smaller tiles give four
+// times the workgroups and waste less on a remainder, the larger ones fewer
+// operand reads and widenings per product.  Measured on 4096 x 12288 (16 / 32
+// row tiles): 16 rows 31.6 / 78.5 us, 64 rows 100 / 107, 96 rows 143 / 156,
+// 128 rows 182 / 160; 12288 x 4096: 96 rows 145 / 167, 128 rows 191 / 175.
+constexpr uint64_t kFewRows = 96;
+
+void launch_project_tiles(hipStream_t s, const uint16_t* x, const uint16_t* w, uint16_t* y, uint64_t rows,
+                          uint64_t in_w, uint64_t out_w, const uint64_t* out_pos) {
+  using namespace exact;
+  constexpr Order kN = Order::kNatural;
+  auto run = [&](auto tile) {
+    using T = decltype(tile);
+    const dim3 grid(static_cast<unsigned>(ceil_div(out_w, T::kOutputs)), static_cast<unsigned>(ceil_div(rows, T::kRows)));
+    k_project_tiles<T><<<grid, T::kThreads, 0, s>>>(x, w, y, rows, in_w, out_w, out_pos);
+  };
+  if (rows == 1 && in_w <= 12288) {  // the input row as FP32 in LDS
+    if (in_w <= 4096 && out_w > 1024)
+      launch_project_row<RowTile<16, 4096>>(s, x, w, y, in_w, out_w, out_pos);
+    else if (in_w <= 4096)
+      launch_project_row<RowTile<32, 4096>>(s, x, w, y, in_w, out_w, out_pos);
+    else
+      launch_project_row<RowTile<32, 12288>>(s, x, w, y, in_w, out_w, out_pos);
+    return;
+  }
+  if (in_w <= 4096 && out_w > 1024) {
+    if (rows <= kFewRows)
+      run(Tile<16, 16, 4, 1, 1, 2, 4, kN, kN>{});
+    else
+      run(Tile<16, 32, 4, 2, 1, 1, 3, kN, kN>{});
+  } else {
+    if (rows <= kFewRows)
+      run(Tile<32, 16, 8, 1, 1, 1, 4, kN, kN>{});
+    else
+      run(Tile<32, 32, 8, 1, 1, 1, 2, kN, kN>{});
+  }
+}
+
 template <class T>
 void launch_projection_rowmajor(hipStream_t s, const void* x, const void* w, void* y, uint64_t rows,
                                 uint64_t in_w, uint64_t out_w, const uint64_t* out_pos) {
@@ -78,6 +309,13 @@ void launch_projection_rowmajor(hipStream_t s, const void* x, const void* w, voi
   const bool narrow = in_w <= 4096 && out_w > 1024;
   const uint64_t row_blocks = ceil_div(rows, RT);
   require(row_blocks <= 65535, "projection rows exceed the launch limit", DL_LENGTH_ERROR);
+  if constexpr (std::is_same_v<T, uint16_t>) {
+    if (tiled_projection(x, w, in_w)) {
+      launch_project_tiles(s, static_cast<const T*>(x), static_cast<const T*>(w), static_cast<T*>(y), rows, in_w, out_w,
+                           out_pos);
+      return;
+    }
+  }
   if (narrow) {
     dim3 grid(grid_for(out_w, kThreads / 16), static_cast<unsigned>(row_blocks));
     projection_rowmajor<T, 16, RT><<<grid, kThreads, 0, s>>>(
@@ -114,7 +352,16 @@ __global__ __launch_bounds__(kThreads) void rms_norm_rows(const T* __restrict__ 
           comp = v * v;
         }
       } else {
-        for (uint64_t col = 4u * t + c; col < width; col += 128) {
+        // Eight loads in flight; the squares add in ascending order.
+        uint64_t col = 4u * t + c;
+        for (; col + 7 * 128 < width; col += 8 * 128) {
+          float v[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) v[k] = load_elem(xr, col + 128 * k);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) comp = comp + v[k] * v[k];
+        }
+        for (; col < width; col += 128) {
           const float v = load_elem(xr, col);
           comp = comp + v * v;
         }

@@ -2510,7 +2510,7 @@ __device__ __forceinline__ u32x2 pack4(const float (&v)[4]) {
 }
 
 template <class T, int EPI>
-__global__ __launch_bounds__(exact::kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_xgemm(XgemmArgs a) {
+__global__ __launch_bounds__(T::kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_xgemm(XgemmArgs a) {
   constexpr int P = T::P, RW = 64 / P;
   if (!a.ctl->active) return;
   // Workgroups are dealt to the XCDs round-robin: XCD x takes the output tiles
@@ -3642,10 +3642,11 @@ void launch_head(dl_plan* p, hipStream_t s, const dl::HeadArgs& a) {
 template <int P, int EPI>
 void launch_xgemm(hipStream_t s, const dl::XgemmArgs& a) {
   using namespace dl::exact;
-  using T = std::conditional_t<P == 16, Tile<16, 4, 2, 1, 3, Order::kPermuted>, Tile<32, 8, 1, 1, 2, Order::kPermuted>>;
+  constexpr Order kP = Order::kPermuted;
+  using T = std::conditional_t<P == 16, Tile<16, 32, 4, 2, 1, 1, 3, kP, kP>, Tile<32, 32, 8, 1, 1, 1, 2, kP, kP>>;
   require(a.N % T::kOutputs == 0 && a.K % T::kInputs == 0 && a.B > 0, "exact GEMM shape");
   const dim3 grid(a.N / T::kOutputs, (a.B + T::kRows - 1) / T::kRows);
-  dl::k_xgemm<T, EPI><<<grid, kThreads, 0, s>>>(a);
+  dl::k_xgemm<T, EPI><<<grid, T::kThreads, 0, s>>>(a);
 }
 
 // The rows one step works on.  For the token loop they are the plan's

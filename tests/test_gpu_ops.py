@@ -52,6 +52,32 @@ def test_projection_rowmajor(device, queue, oracle, rows, in_w, out_w):
     assert np.array_equal(down(queue, by, np.uint16, rows * out_w), oracle.projection(x, w, rows, in_w, out_w))
 
 
+@pytest.mark.parametrize("rows,in_w,out_w", [(2, 256, 33), (15, 256, 1025), (16, 512, 1040), (17, 768, 1025),
+                                             (16, 4352, 1040), (17, 4352, 47), (31, 256, 64), (33, 4096, 1088),
+                                             (33, 4096, 96), (96, 512, 1040), (65, 256, 1027), (3, 1280, 5),
+                                             (97, 256, 1027), (97, 4352, 47), (130, 384 * 2, 1088), (129, 512, 96),
+                                             (1, 256, 5), (1, 256, 1030), (1, 1280, 1025), (1, 4352, 47),
+                                             (1, 12288, 33), (1, 12544, 33)])
+def test_projection_row_tiles(device, queue, oracle, rows, in_w, out_w):
+    """Row counts, output widths and stage counts around the one-row kernel
+    and the matrix-core tiles (16 and 32 rows; 8, 16, 32 and 64 outputs; fewer
+    stages than buffers), the output at a device position, and the same values
+    from operands that are not 16-byte aligned (the general path)."""
+    rng = np.random.default_rng(rows * 131 + in_w + out_w)
+    x = oracle.bf16_from_f32(rng.standard_normal(rows * in_w).astype(np.float32))
+    w = oracle.bf16_from_f32((0.05 * rng.standard_normal(out_w * in_w)).astype(np.float32))
+    want = oracle.projection(x, w, rows, in_w, out_w)
+    bpos = up(device, queue, np.array([3], np.uint64))
+    for shift in (0, 1):
+        pad = np.zeros(shift, np.uint16)
+        bx, bw = up(device, queue, np.concatenate([pad, x])), up(device, queue, np.concatenate([pad, w]))
+        by = up(device, queue, np.full((rows + 4) * out_w, 0x7fc0, np.uint16))
+        run_op(queue, "dl_projection", 1, bx.ptr(2 * shift), bw.ptr(2 * shift), by.ptr(), rows, in_w, out_w, bpos.ptr())
+        got = down(queue, by, np.uint16, (rows + 4) * out_w)
+        assert np.array_equal(got[3 * out_w:(rows + 3) * out_w], want), shift
+        assert np.all(got[:3 * out_w] == 0x7fc0) and np.all(got[(rows + 3) * out_w:] == 0x7fc0)
+
+
 @pytest.mark.parametrize("in_w,out_w", [(4096, 4096), (4096, 1024), (4096, 12288), (12288, 4096), (4096, 16384),
                                         (256, 2048), (512, 64)])
 def test_projection_packed(device, queue, oracle, in_w, out_w):
