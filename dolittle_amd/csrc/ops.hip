@@ -511,6 +511,160 @@ __global__ __launch_bounds__(kThreads) void attention_retained(
   }
 }
 
+// 16 consecutive features in FP32; 16-byte aligned.
+__device__ __forceinline__ void load_features(const uint16_t* p, float (&v)[16]) {
+  const u32x4* q = reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const u32x4 w = q[i];
+    v[8 * i + 0] = dl_bf16_lo(w.x); v[8 * i + 1] = dl_bf16_hi(w.x);
+    v[8 * i + 2] = dl_bf16_lo(w.y); v[8 * i + 3] = dl_bf16_hi(w.y);
+    v[8 * i + 4] = dl_bf16_lo(w.z); v[8 * i + 5] = dl_bf16_hi(w.z);
+    v[8 * i + 6] = dl_bf16_lo(w.w); v[8 * i + 7] = dl_bf16_hi(w.w);
+  }
+}
+__device__ __forceinline__ void load_features(const float* p, float (&v)[16]) {
+  const float4* q = reinterpret_cast<const float4*>(p);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 w = q[i];
+    v[4 * i] = w.x; v[4 * i + 1] = w.y; v[4 * i + 2] = w.z; v[4 * i + 3] = w.w;
+  }
+}
+
+// attention_retained for heads of 128 features on 16-byte aligned rows: the
+// same ranges, merges and rounding points (attention.cu:231-383) with the
+// latencies overlapped.  Every thread keeps several key rows in flight, all
+// threads take part in the exponentials, and the two PV chains of a feature
+// read 16 keys ahead.  One workgroup per (position, query head), numbered so
+// that the heads of a K/V group run on one XCD.  Bound: at one row the issue
+// of the chains' instructions (load, widening, FMA per key); 16 rows at 1024
+// keys 321 -> 43 us, one row at 512 keys 138 -> 24 us, at 4000 keys 107 us.
+constexpr int kRowThreads = 512;
+constexpr int kHeadWidth = 128;
+
+template <class T>
+__global__ __launch_bounds__(kRowThreads) void attention_heads(const T* __restrict__ q, const T* __restrict__ k,
+                                                               const T* __restrict__ v, T* __restrict__ out,
+                                                               uint64_t tasks, uint32_t q_heads, uint32_t kv_heads,
+                                                               uint64_t host_first, const float* scale_ptr,
+                                                               const uint64_t* dev_pos) {
+  extern __shared__ __align__(16) float scores[];
+  __shared__ float wave_values[kRowThreads / 64];
+  __shared__ float denominator_shared;
+  __shared__ float halves[2 * kHeadWidth];
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int part = tid % 8, group = tid / 8;  // 8 lanes per key, 16 features each
+  const uint32_t ratio = q_heads / kv_heads;
+  const uint64_t stride = static_cast<uint64_t>(kv_heads) * kHeadWidth;
+  const float scale = *scale_ptr;
+  const uint64_t first = position_or(dev_pos, host_first);
+  for (uint64_t id = blockIdx.x; id < tasks; id += gridDim.x) {
+    const uint32_t in_row = static_cast<uint32_t>(id % q_heads);
+    const uint32_t kvh = in_row % kv_heads;
+    const uint64_t task = id - in_row + kvh * ratio + in_row / kv_heads;
+    const int count = static_cast<int>(first + id / q_heads + 1);
+    const T* krow = k + static_cast<uint64_t>(kvh) * kHeadWidth + 16 * part;
+    float qv[16];
+    load_features(q + task * kHeadWidth + 16 * part, qv);
+    constexpr int kKeys = kRowThreads / 8, kAhead = 4;
+    float maximum = -INFINITY;
+    // The maximum over the thread's own scores; a NaN score is ignored, as
+    // fmaxf does in any order.
+    for (int base = 0; base < count; base += kAhead * kKeys) {
+      float kv[kAhead][16];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+        load_features(krow + static_cast<uint64_t>(min(base + i * kKeys + group, count - 1)) * stride, kv[i]);
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const int j = base + i * kKeys + group;
+        float partial = 0.0f;
+#pragma unroll
+        for (int f = 0; f < 16; ++f) partial = fma_rn(qv[f], kv[i][f], partial);
+        partial = partial + row_down<4>(partial);
+        partial = partial + row_down<2>(partial);
+        partial = partial + row_down<1>(partial);
+        if (part == 0 && j < count) {
+          const float s = partial * scale;
+          scores[j] = s;
+          maximum = fmaxf(maximum, s);
+        }
+      }
+    }
+    maximum = wave_max(maximum);
+    if (lane == 0) wave_values[wave] = maximum;
+    __syncthreads();
+    // The reference starts the maximum from score 0: a row of NaN keeps it.
+    maximum = scores[0];
+#pragma unroll
+    for (int w = 0; w < kRowThreads / 64; ++w) maximum = fmaxf(maximum, wave_values[w]);
+    __syncthreads();
+    for (int j = tid; j < count; j += kRowThreads) scores[j] = dl_expf(scores[j] - maximum);
+    __syncthreads();
+    if (tid < 32) {
+      float partial = 0.0f;
+      int j = tid;
+      for (; j + 15 * 32 < count; j += 16 * 32) {
+        float e[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) e[i] = scores[j + 32 * i];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) partial = partial + e[i];
+      }
+      for (; j < count; j += 32) partial = partial + scores[j];
+#pragma unroll
+      for (int off = 16; off; off >>= 1) partial = partial + __shfl_down(partial, off, 32);
+      if (tid == 0) denominator_shared = partial;
+    }
+    __syncthreads();
+    const float denominator = denominator_shared;
+    for (int j = tid; j < count; j += kRowThreads) scores[j] = scores[j] / denominator;
+    __syncthreads();
+    if (tid < 2 * kHeadWidth) {
+      const int split = (count - 1) / 2 + 1, feature = tid % kHeadWidth, half = tid / kHeadWidth;
+      const int end = half ? count : split;
+      const T* vrow = v + static_cast<uint64_t>(kvh) * kHeadWidth + feature;
+      float sum = 0.0f;
+      int j = half ? split : 0;
+      for (; j < end && j % 4; ++j) sum = fma_rn(scores[j], load_elem(vrow, j * stride), sum);
+      constexpr int kBatch = 16;
+      T va[kBatch], vb[kBatch];
+      auto load = [&](T (&x)[kBatch], int at) {  // past the range: its last key again
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) x[i] = vrow[static_cast<uint64_t>(min(at + i, end - 1)) * stride];
+      };
+      auto chain = [&](const T (&x)[kBatch], int at) {
+#pragma unroll
+        for (int i = 0; i < kBatch; i += 4) {
+          const float4 p = *reinterpret_cast<const float4*>(scores + at + i);
+          sum = fma_rn(p.x, load_elem(x, i), sum);
+          sum = fma_rn(p.y, load_elem(x, i + 1), sum);
+          sum = fma_rn(p.z, load_elem(x, i + 2), sum);
+          sum = fma_rn(p.w, load_elem(x, i + 3), sum);
+        }
+      };
+      const int batches = (end - j) / kBatch;
+      if (batches > 0) load(va, j);
+      for (int b = 0; b < batches; b += 2) {
+        load(vb, j + kBatch);
+        chain(va, j);
+        j += kBatch;
+        if (b + 1 < batches) {
+          load(va, j + kBatch);
+          chain(vb, j);
+          j += kBatch;
+        }
+      }
+      for (; j < end; ++j) sum = fma_rn(scores[j], load_elem(vrow, j * stride), sum);
+      halves[tid] = sum;
+    }
+    __syncthreads();
+    if (tid < kHeadWidth) store_elem(out, task * kHeadWidth + tid, halves[tid] + halves[tid + kHeadWidth]);
+    __syncthreads();
+  }
+}
+
 // -------------------------------------------------------- embedding, add, silu
 // embedding.cu:60-80; a token outside the table writes zeros instead of
 // reading out of bounds.
@@ -644,7 +798,21 @@ int dl_attention(dl_queue* queue, int dtype, const void* query, const void* key,
             DL_LENGTH_ERROR);
     const uint64_t tasks = positions * query_heads;
     const unsigned grid = dl::grid_for(tasks, 1, 65535);
-    if (dtype == DL_BF16)
+    const bool aligned = (reinterpret_cast<uintptr_t>(query) | reinterpret_cast<uintptr_t>(key) |
+                          reinterpret_cast<uintptr_t>(value)) % 16 == 0;
+    if (width == dl::kHeadWidth && aligned && query_heads <= UINT32_MAX) {
+      auto run = [&](auto tag) {
+        using T = decltype(tag);
+        dl::attention_heads<T><<<grid, dl::kRowThreads, shared_bytes, queue->stream>>>(
+            static_cast<const T*>(query), static_cast<const T*>(key), static_cast<const T*>(value),
+            static_cast<T*>(output), tasks, static_cast<uint32_t>(query_heads), static_cast<uint32_t>(kv_heads),
+            first_position, scale, device_position);
+      };
+      if (dtype == DL_BF16)
+        run(uint16_t{});
+      else
+        run(float{});
+    } else if (dtype == DL_BF16)
       dl::attention_retained<uint16_t><<<grid, dl::kThreads, shared_bytes, queue->stream>>>(
           static_cast<const uint16_t*>(query), static_cast<const uint16_t*>(key),
           static_cast<const uint16_t*>(value), static_cast<uint16_t*>(output), tasks, query_heads,

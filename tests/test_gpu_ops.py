@@ -133,6 +133,29 @@ def test_attention(device, queue, oracle, rows, first):
     assert np.array_equal(down(queue, by, np.uint16, q.size), oracle.attention(q, k, v, rows, hq, hkv, width, first))
 
 
+@pytest.mark.parametrize("rows,first", [(1, 2), (1, 6), (2, 30), (3, 33), (1, 63), (1, 64), (1, 127), (2, 255),
+                                        (5, 511), (1, 513)])
+@pytest.mark.parametrize("hq,hkv", [(4, 2), (3, 3)])
+def test_attention_key_counts(device, queue, oracle, rows, first, hq, hkv):
+    """Key counts around the 128-feature kernel's passes (64 keys, four passes
+    in flight) and PV batches (16 keys from an aligned key), and the same
+    values from operands that are not 16-byte aligned (the general kernel)."""
+    width, total = 128, first + rows
+    rng = np.random.default_rng(total * 7 + hq)
+    q, k, v = (oracle.bf16_from_f32(rng.standard_normal(n * width).astype(np.float32))
+               for n in (rows * hq, total * hkv, total * hkv))
+    want = oracle.attention(q, k, v, rows, hq, hkv, width, first)
+    scale = device.allocate(4)
+    run_op(queue, "dl_attention_scale", scale.ptr(), width)
+    bpos = up(device, queue, np.array([first], np.uint64))
+    for shift in (0, 1):
+        bq, bk, bv = (up(device, queue, np.concatenate([np.zeros(shift, np.uint16), a])) for a in (q, k, v))
+        by = device.allocate(q.nbytes)
+        run_op(queue, "dl_attention", 1, bq.ptr(2 * shift), bk.ptr(2 * shift), bv.ptr(2 * shift), by.ptr(), rows, hq, hkv,
+               width, 0, bpos.ptr(), total, scale.ptr())
+        assert np.array_equal(down(queue, by, np.uint16, q.size), want), shift
+
+
 def test_attention_reference_operands(device, queue, oracle):
     """operator_reference.cpp:273-313 shapes: 4 heads, 2 KV heads, width 128."""
     for rows in (1, 37):
