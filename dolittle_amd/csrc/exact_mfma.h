@@ -61,6 +61,13 @@ struct Tile {
   static_assert(kRing >= 2 && kRing <= 4, "two to four stage buffers");
 };
 
+// Rows up to which 16-row tiles beat 32-row ones: they give four times the
+// workgroups and waste less on a remainder, the larger ones need fewer operand
+// reads and widenings per product.  Row-major 4096 x 12288 (16 / 32 row tiles):
+// 16 rows 31.6 / 78.5 us, 64 rows 100 / 107, 96 rows 143 / 156, 128 rows 182 /
+// 160; 12288 x 4096: 96 rows 145 / 167, 128 rows 191 / 175.
+constexpr uint64_t kTileFewRows = 96;
+
 // s_waitcnt immediates: at most n vector-memory operations outstanding (vmcnt
 // bits 3:0 and 15:14; expcnt and lgkmcnt at their no-wait maxima); the same
 // and no LDS operation outstanding.

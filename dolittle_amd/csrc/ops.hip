@@ -264,13 +264,6 @@ bool tiled_projection(const void* x, const void* w, uint64_t in_w) {
   return in_w % 256 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
 }
 
-// Tiles of 16 rows up to kFewRows, of 32 above: the smaller tiles give four
-// times the workgroups and waste less on a remainder, the larger ones fewer
-// operand reads and widenings per product.  Measured on 4096 x 12288 (16 / 32
-// row tiles): 16 rows 31.6 / 78.5 us, 64 rows 100 / 107, 96 rows 143 / 156,
-// 128 rows 182 / 160; 12288 x 4096: 96 rows 145 / 167, 128 rows 191 / 175.
-constexpr uint64_t kFewRows = 96;
-
 void launch_project_tiles(hipStream_t s, const uint16_t* x, const uint16_t* w, uint16_t* y, uint64_t rows,
                           uint64_t in_w, uint64_t out_w, const uint64_t* out_pos) {
   using namespace exact;
@@ -290,12 +283,12 @@ void launch_project_tiles(hipStream_t s, const uint16_t* x, const uint16_t* w, u
     return;
   }
   if (in_w <= 4096 && out_w > 1024) {
-    if (rows <= kFewRows)
+    if (rows <= kTileFewRows)
       run(Tile<16, 16, 4, 1, 1, 2, 4, kN, kN>{});
     else
       run(Tile<16, 32, 4, 2, 1, 1, 3, kN, kN>{});
   } else {
-    if (rows <= kFewRows)
+    if (rows <= kTileFewRows)
       run(Tile<32, 16, 8, 1, 1, 1, 4, kN, kN>{});
     else
       run(Tile<32, 32, 8, 1, 1, 1, 2, kN, kN>{});

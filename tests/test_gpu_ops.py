@@ -95,6 +95,29 @@ def test_projection_packed(device, queue, oracle, in_w, out_w):
     assert np.array_equal(down(queue, by, np.uint16, out_w), oracle.projection(x, w, 1, in_w, out_w))
 
 
+@pytest.mark.parametrize("rows,in_w,out_w", [(2, 128, 1028), (3, 384, 2048), (16, 512, 1028), (17, 256, 34),
+                                             (97, 384, 1028), (97, 256, 34), (5, 4352, 66)])
+def test_projection_packed_rows(device, queue, oracle, rows, in_w, out_w):
+    """Several rows around the matrix-core tiles (and one stage of inputs),
+    the output at a device position, and the same values from input rows that
+    are not 16-byte aligned (one row per launch)."""
+    from dolittle_amd import _lib
+    rng = np.random.default_rng(rows * 17 + in_w + out_w)
+    x = oracle.bf16_from_f32(rng.standard_normal(rows * in_w).astype(np.float32))
+    w = oracle.bf16_from_f32((0.05 * rng.standard_normal(out_w * in_w)).astype(np.float32))
+    want = oracle.projection(x, w, rows, in_w, out_w)
+    bw, packed = up(device, queue, w), device.allocate(out_w * in_w * 2)
+    run_op(queue, "dl_projection_pack", bw.ptr(), packed.ptr(), out_w, in_w)
+    bpos = up(device, queue, np.array([2], np.uint64))
+    for shift in (0, 1):
+        bx = up(device, queue, np.concatenate([np.zeros(shift, np.uint16), x]))
+        by = up(device, queue, np.full((rows + 3) * out_w, 0x7fc0, np.uint16))
+        run_op(queue, "dl_projection_packed", bx.ptr(2 * shift), packed.ptr(), by.ptr(), rows, in_w, out_w, bpos.ptr())
+        got = down(queue, by, np.uint16, (rows + 3) * out_w)
+        assert np.array_equal(got[2 * out_w:(rows + 2) * out_w], want), shift
+        assert np.all(got[:2 * out_w] == 0x7fc0) and np.all(got[(rows + 2) * out_w:] == 0x7fc0)
+
+
 @pytest.mark.parametrize("first", [0, 1, 511, 4093, 8191])
 def test_rotary(device, queue, oracle, first):
     rows, heads, width = 3, 2, 128
