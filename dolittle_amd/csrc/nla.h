@@ -14,25 +14,67 @@ namespace dl::nla {
 constexpr unsigned kLanes = 8;      // strided partial sums of the reference reduction
 constexpr unsigned kThreads = 256;  // one workgroup per vector operation
 
+constexpr uint64_t kChunk = 4096;   // squares in LDS at a time
+constexpr int kBatch = 8;           // values a thread has in flight
+
+// f(i, load(i)) for the indices i = first + threadIdx.x + k * blockDim.x below
+// `end`, kBatch loads ahead of the calls that use them.
+template <class Load, class F>
+__device__ __forceinline__ void for_each_loaded(uint64_t first, uint64_t end, Load&& load, F&& f) {
+  for (uint64_t base = first + threadIdx.x; base < end; base += kBatch * blockDim.x) {
+    decltype(load(base)) v[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const uint64_t i = base + k * blockDim.x;
+      v[k] = load(i < end ? i : base);
+    }
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const uint64_t i = base + k * blockDim.x;
+      if (i < end) f(i, v[k]);
+    }
+  }
+}
+
 // sum_i value(i)^2 in the reference order: lane k < 8 accumulates
 // i = k, k + 8, k + 16, ... ascending, with separately rounded multiply and
 // add; thread 0 then adds lanes 0..7 left to right.  Every thread of the
-// workgroup calls; all receive the sum (kept in sums[kLanes]).
-template <class F>
-__device__ __forceinline__ float square_sum(uint64_t width, F&& value, float* sums) {
-  if (threadIdx.x < kLanes) {
-    float sum = 0.0f;
-    for (uint64_t i = threadIdx.x; i < width; i += kLanes) {
-      const float v = value(i);
-      sum = __fadd_rn(sum, __fmul_rn(v, v));
+// workgroup calls; all receive the sum (kept in sums[kLanes]).  The whole
+// workgroup loads and squares into LDS and the eight lanes only add from
+// there, 16 reads ahead (with eight threads loading as they add, a 4096-wide
+// row waited for 512 memory latencies in turn: 40-56 us per operation, now
+// 8).  value(load(i)) may have side effects: it runs once per index.
+template <class Load, class F>
+__device__ __forceinline__ float square_sum(uint64_t width, Load&& load, F&& value, float* sums) {
+  __shared__ float squares[kChunk];
+  float sum = 0.0f;
+  for (uint64_t base = 0; base < width; base += kChunk) {
+    const int n = static_cast<int>(width - base < kChunk ? width - base : kChunk);
+    for_each_loaded(base, base + n, load, [&](uint64_t i, auto raw) {
+      const float v = value(raw);
+      squares[i - base] = __fmul_rn(v, v);
+    });
+    __syncthreads();
+    if (threadIdx.x < kLanes) {
+      constexpr int kAhead = 16;
+      int i = threadIdx.x;
+      for (; i + (kAhead - 1) * static_cast<int>(kLanes) < n; i += kAhead * kLanes) {
+        float s[kAhead];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) s[k] = squares[i + k * kLanes];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) sum = __fadd_rn(sum, s[k]);
+      }
+      for (; i < n; i += kLanes) sum = __fadd_rn(sum, squares[i]);
     }
-    sums[threadIdx.x] = sum;
+    __syncthreads();
   }
+  if (threadIdx.x < kLanes) sums[threadIdx.x] = sum;
   __syncthreads();
   if (threadIdx.x == 0) {
-    float sum = 0.0f;
-    for (unsigned k = 0; k < kLanes; ++k) sum = __fadd_rn(sum, sums[k]);
-    sums[kLanes] = sum;
+    float total = 0.0f;
+    for (unsigned k = 0; k < kLanes; ++k) total = __fadd_rn(total, sums[k]);
+    sums[kLanes] = total;
   }
   __syncthreads();
   return sums[kLanes];
@@ -55,7 +97,8 @@ __device__ __forceinline__ void intervene_row(T* row, const float* direction, ui
     state[1] = state[1] + 1;
   }
   __syncthreads();
-  const float sum = square_sum(width, [&](uint64_t i) { return load_elem(row, i); }, sums);
+  auto load = [&](uint64_t i) { return load_elem(row, i); };
+  const float sum = square_sum(width, load, [](float v) { return v; }, sums);
   if (threadIdx.x == 0) {
     const float beta = __fmul_rn(strength, __builtin_sqrtf(sum));
     sums[kLanes + 1] = beta;
@@ -66,11 +109,13 @@ __device__ __forceinline__ void intervene_row(T* row, const float* direction, ui
   const bool valid = *invalid == 0;
   __syncthreads();
   if (valid) {
-    for (uint64_t i = threadIdx.x; i < width; i += blockDim.x) {
-      const float value = __fadd_rn(load_elem(row, i), __fmul_rn(beta, direction[i]));
-      store_elem(row, i, value);
-      if (!finite(value) || !finite(storage_round<T>(value))) atomicOr(invalid, 1u);
-    }
+    for_each_loaded(
+        0, width, [&](uint64_t i) { return float2{load_elem(row, i), direction[i]}; },
+        [&](uint64_t i, float2 v) {
+          const float value = __fadd_rn(v.x, __fmul_rn(beta, v.y));
+          store_elem(row, i, value);
+          if (!finite(value) || !finite(storage_round<T>(value))) atomicOr(invalid, 1u);
+        });
   }
   __syncthreads();
   if (threadIdx.x == 0) state[0] = *invalid;

@@ -28,8 +28,8 @@ __global__ __launch_bounds__(kThreads) void k_inject(const In* source, Out* outp
   __shared__ uint32_t invalid;
   if (threadIdx.x == 0) invalid = 0;
   __syncthreads();
-  const float sum = square_sum(width, [&](uint64_t i) {
-    const float v = load_elem(source, i);
+  auto load = [&](uint64_t i) { return load_elem(source, i); };
+  const float sum = square_sum(width, load, [&](float v) {
     if (!finite(v)) atomicOr(&invalid, 1u);
     return v;
   }, sums);
@@ -44,11 +44,11 @@ __global__ __launch_bounds__(kThreads) void k_inject(const In* source, Out* outp
   const bool valid = invalid == 0;  // before any output latch below
   __syncthreads();
   if (valid) {
-    for (uint64_t i = threadIdx.x; i < width; i += blockDim.x) {
-      const float value = __fmul_rn(__fdiv_rn(load_elem(source, i), n), scale);
+    for_each_loaded(0, width, load, [&](uint64_t i, float v) {
+      const float value = __fmul_rn(__fdiv_rn(v, n), scale);
       store_elem(output, i, value);
       if (!finite(value) || !finite(storage_round<Out>(value))) atomicOr(&invalid, 1u);
-    }
+    });
   }
   __syncthreads();
   if (threadIdx.x == 0) *status = invalid;
@@ -61,9 +61,8 @@ template <class In>
 __global__ __launch_bounds__(kThreads) void k_direction(const In* original, const In* edited, float* direction,
                                                          uint32_t* status, uint64_t width) {
   __shared__ float sums[kLanes + 2];
-  const float sum = square_sum(width, [&](uint64_t i) {
-    return __fsub_rn(load_elem(edited, i), load_elem(original, i));
-  }, sums);
+  auto load = [&](uint64_t i) { return __fsub_rn(load_elem(edited, i), load_elem(original, i)); };
+  const float sum = square_sum(width, load, [](float v) { return v; }, sums);
   if (threadIdx.x == 0) {
     const float n = __builtin_sqrtf(sum);
     sums[kLanes + 1] = n;
@@ -72,8 +71,7 @@ __global__ __launch_bounds__(kThreads) void k_direction(const In* original, cons
   __syncthreads();
   const float n = sums[kLanes + 1];
   if (!finite(n) || n == 0.0f) return;
-  for (uint64_t i = threadIdx.x; i < width; i += blockDim.x)
-    direction[i] = __fdiv_rn(__fsub_rn(load_elem(edited, i), load_elem(original, i)), n);
+  for_each_loaded(0, width, load, [&](uint64_t i, float v) { direction[i] = __fdiv_rn(v, n); });
 }
 
 __global__ void k_intervention_reset(uint32_t* state) {

@@ -140,3 +140,35 @@ def test_intervention_overflow_latches(device, queue, oracle):
     assert state[0] == 1
     assert queue.read(iv.state, np.uint32, 2).tolist() == state.tolist()
     assert np.array_equal(queue.read(bh, np.uint16, width), expect)
+
+
+@pytest.mark.parametrize("width", [2, 9, 127, 129, 2047, 2049, 4097, 8199])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_row_widths_match_oracle(device, queue, oracle, width, bf16):
+    """Widths around the eight lanes, the values a thread holds in flight and
+    the chunks of squares kept on chip, for the three operations."""
+    from dolittle_amd.interventions import DeviceDirection, DeviceInjection, DeviceIntervention
+    kind = "bfloat16" if bf16 else "float32"
+    x, e = source(oracle, width, width, bf16), source(oracle, width, width + 1, bf16)
+    bx, be = up(device, queue, x), up(device, queue, e)
+    inj = DeviceInjection(device, queue, region(bx, x.nbytes), kind, kind, width, 7.5)
+    inj.submit()
+    queue.drain()
+    status, norm, out = oracle.inject(x, bf16, bf16, 7.5)
+    raw = queue.read(inj.storage, np.uint8, inj.storage.nbytes)
+    assert raw[4:8].view(np.uint32)[0] == status and raw[0:4].view(np.float32)[0] == norm
+    assert np.array_equal(raw[8:].view(x.dtype), out)
+    d = DeviceDirection(device, queue, region(bx, x.nbytes), region(be, e.nbytes), kind, width)
+    d.submit()
+    u = d.finish()
+    _, direction = oracle.direction(x, e, bf16)
+    assert np.array_equal(queue.read(u.owner, np.float32, width, u.offset), direction)
+    pos = up(device, queue, np.array([5], np.uint64))
+    iv = DeviceIntervention(device, queue, u, width, 5, 0.37, kind)
+    iv.initialize()
+    iv.submit(region(bx, x.nbytes), region(pos, 8), 1)
+    queue.drain()
+    state, expect = np.zeros(2, np.uint32), x.copy()
+    assert oracle.intervene(expect, bf16, 1, width, direction, 5, 5, 0.37, state)
+    assert np.array_equal(queue.read(bx, x.dtype, width), expect)
+    assert queue.read(iv.state, np.uint32, 2).tolist() == state.tolist() == [0, 1]
