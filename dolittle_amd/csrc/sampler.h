@@ -35,8 +35,9 @@
 namespace dl::sampling {
 
 constexpr int kBins = 65536;
-constexpr int kCountBlocks = 64;
-constexpr int kCountThreads = 256;
+constexpr int kCountBlocks = 64;  // argmax partials a row has room for
+constexpr int kCountParts = 16;   // workgroups per row of the counting pass
+constexpr int kCountThreads = 1024;
 constexpr int kSelectThreads = 1024;
 constexpr int kBinsPerThread = kBins / kSelectThreads;
 constexpr int kMtWords = 312;

@@ -6,11 +6,12 @@
 //                  argmax partials (largest value, lowest id) and, for
 //                  categorical rows, the per-value histogram over the 16-bit
 //                  order key (descending value == descending key; -0 joins +0)
-// k_sample_select  one 1024-lane workgroup per row: FP64 weight per distinct
-//                  value, prefix estimates, guarded cutoff and draw decisions
-//                  (exact serial replay when a decision falls inside the error
-//                  band), id lookup of the chosen value's j-th occurrence, and
-//                  the histogram cleared for the next selection
+// k_sample_select  one 1024-lane workgroup per row: the distinct values
+//                  compacted, FP64 weight per distinct value, prefix estimates,
+//                  guarded cutoff and draw decisions (exact serial replay when
+//                  a decision falls inside the error band), id lookup of the
+//                  chosen value's j-th occurrence, and the histogram cleared for
+//                  the next selection
 //
 // Error band.  Let E_k be the exact sum of the first k weights.  The host
 // fold F_k differs from E_k by at most (k - 1) * 2^-53 * E_k (positive
@@ -36,7 +37,6 @@ namespace dl::sampling {
 namespace {
 
 constexpr uint32_t kNone = 0xffffffffu;
-constexpr int kLookupTile = kSelectThreads * 16;
 constexpr uint64_t kMtUpper = 0xffffffff80000000ull;
 constexpr uint64_t kMtLower = 0x7fffffffull;
 constexpr uint64_t kMtMatrix = 0xb5026f5aa96619e9ull;
@@ -182,7 +182,13 @@ __device__ __forceinline__ bool row_live(const RowsArgs& a, int row) {
 }
 
 // ------------------------------------------------------------- counting
+// A workgroup counts its part of a row in LDS, two 16-bit counts per word (at
+// most 65535 ids at a time, so none overflows), and adds only the values that
+// occur to the row's histogram: a 151,936-id row of a random model costs about
+// 16 x 2,500 device-scope atomics instead of one per id (48 -> 12 us; they
+// serialize where ids share a value).
 __global__ __launch_bounds__(kCountThreads) void k_sample_count(RowsArgs a) {
+  __shared__ __align__(16) uint32_t bins[kBins / 2];
   __shared__ uint64_t wave_keys[kCountThreads / 64];
   __shared__ uint32_t wave_flags[kCountThreads / 64];
   // Consecutive workgroups go to different XCDs; taking the row from the
@@ -192,22 +198,52 @@ __global__ __launch_bounds__(kCountThreads) void k_sample_count(RowsArgs a) {
   if (!row_live(a, row)) return;
   const bool categorical = a.settings.mode == 1;
   const uint16_t* x = a.logits + static_cast<uint64_t>(row) * a.row_stride;
-  const uint32_t chunk = (a.n + kCountBlocks - 1) / kCountBlocks;
+  const uint32_t chunk = (a.n + kCountParts - 1) / kCountParts;
   const uint32_t begin = min(a.n, static_cast<uint32_t>(part) * chunk);
   const uint32_t end = min(a.n, begin + chunk);
   uint32_t* hist = a.ws.hist + static_cast<uint64_t>(row) * kBins;
+  u32x4* quads = reinterpret_cast<u32x4*>(bins);
+  constexpr int kQuads = kBins / 8, kAhead = 8;
+  constexpr uint32_t kMost = 65535;
   uint64_t best = 0;
   uint32_t flags = 0;
-  for (uint32_t i = begin + threadIdx.x; i < end; i += kCountThreads) {
-    const uint32_t v = x[i];
-    if (bf16_rejected(v)) {
-      flags |= 1u;
-    } else if (bf16_is_finite(v)) {
-      flags |= 2u;
-      const uint32_t key = bf16_order(v);
-      const uint64_t k = (static_cast<uint64_t>(key) << 32) | (0xffffffffu - i);
-      best = k > best ? k : best;
-      if (categorical) atomicAdd(hist + key, 1u);
+  for (uint32_t first = begin; first < end; first += kMost) {
+    const uint32_t last = min(end, first + kMost);
+    if (categorical) {
+      for (int i = threadIdx.x; i < kQuads; i += kCountThreads) quads[i] = u32x4{0u, 0u, 0u, 0u};
+      __syncthreads();
+    }
+    for (uint32_t base = first + threadIdx.x; base < last; base += kAhead * kCountThreads) {
+      uint16_t v[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) v[k] = x[min(base + k * kCountThreads, last - 1)];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const uint32_t i = base + k * kCountThreads;
+        if (i >= last) break;
+        if (bf16_rejected(v[k])) {
+          flags |= 1u;
+        } else if (bf16_is_finite(v[k])) {
+          flags |= 2u;
+          const uint32_t key = bf16_order(v[k]);
+          const uint64_t packed = (static_cast<uint64_t>(key) << 32) | (0xffffffffu - i);
+          best = packed > best ? packed : best;
+          if (categorical) atomicAdd(&bins[key / 2], (key & 1u) ? 0x10000u : 1u);
+        }
+      }
+    }
+    if (categorical) {
+      __syncthreads();
+      for (int i = threadIdx.x; i < kQuads; i += kCountThreads) {
+        const u32x4 q = quads[i];
+        const uint32_t words[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (words[j] & 0xffffu) atomicAdd(hist + 8 * i + 2 * j, words[j] & 0xffffu);
+          if (words[j] >> 16) atomicAdd(hist + 8 * i + 2 * j + 1, words[j] >> 16);
+        }
+      }
+      __syncthreads();
     }
   }
   best = wave_max_u64(best);
@@ -240,36 +276,48 @@ __device__ __forceinline__ bool reaches(double v, double threshold, bool strict)
   return strict ? v > threshold : v >= threshold;
 }
 
-// First kept candidate in this thread's bins whose prefix estimate reaches
-// `threshold`.  The estimates form this thread's canonical non-decreasing
-// sequence: A starts at the thread's scanned prefix, grows by count * weight
-// per bin, and candidate j of a bin is estimated as A + j * weight.
-__device__ __forceinline__ Found walk(const uint32_t (&count)[kBinsPerThread], uint32_t top, double A,
-                                      uint32_t k, uint32_t kept_left, const double* w_row, double threshold,
-                                      bool strict) {
-  int hit = -1;
+// kBatch consecutive distinct values of a thread.
+constexpr int kBatch = 8;
+struct Batch {
+  uint32_t key[kBatch], count[kBatch];
+  double weight[kBatch];
+};
+
+// First kept candidate among this thread's values whose prefix estimate
+// reaches `threshold`.  The estimates form this thread's canonical
+// non-decreasing sequence: A starts at the thread's scanned prefix, grows by
+// count * weight per value, and candidate j of a value is estimated as A + j *
+// weight.  batch(b) gives the thread's b-th batch; counts of values past its
+// last are zero.
+template <class BatchOf>
+__device__ __forceinline__ Found walk(int batches, BatchOf&& batch, double A, uint32_t k, uint32_t kept_left,
+                                      double threshold, bool strict) {
+  bool found = false;
   double hit_a = 0.0, hit_w = 0.0;
-  uint32_t hit_k = 0, hit_count = 0;
+  uint32_t hit_k = 0, hit_count = 0, hit_key = 0;
+  for (int b = 0; b < batches && !found; ++b) {
+    const Batch& v = batch(b);
 #pragma unroll
-  for (int q = 0; q < kBinsPerThread; ++q) {
-    const uint32_t kq = min(count[q], kept_left);
-    kept_left -= kq;
-    if (kq && hit < 0) {
-      const double w = w_row[top - q];
-      const double end = A + static_cast<double>(kq) * w;
-      if (reaches(end, threshold, strict)) {
-        hit = q;
-        hit_a = A;
-        hit_w = w;
-        hit_k = k;
-        hit_count = kq;
-      } else {
-        A = end;
-        k += kq;
+    for (int q = 0; q < kBatch; ++q) {
+      const uint32_t kq = min(v.count[q], kept_left);
+      kept_left -= kq;
+      if (kq && !found) {
+        const double end = A + static_cast<double>(kq) * v.weight[q];
+        if (reaches(end, threshold, strict)) {
+          found = true;
+          hit_a = A;
+          hit_w = v.weight[q];
+          hit_k = k;
+          hit_count = kq;
+          hit_key = v.key[q];
+        } else {
+          A = end;
+          k += kq;
+        }
       }
     }
   }
-  if (hit < 0) return Found{kNone, 0, 0, 0.0};
+  if (!found) return Found{kNone, 0, 0, 0.0};
   uint32_t lo = 1, hi = hit_count;
   while (lo < hi) {
     const uint32_t mid = lo + (hi - lo) / 2;
@@ -278,7 +326,7 @@ __device__ __forceinline__ Found walk(const uint32_t (&count)[kBinsPerThread], u
     else
       lo = mid + 1;
   }
-  return Found{hit_k + lo, top - static_cast<uint32_t>(hit), lo, hit_a + static_cast<double>(lo) * hit_w};
+  return Found{hit_k + lo, hit_key, lo, hit_a + static_cast<double>(lo) * hit_w};
 }
 
 // The host law folded serially over the histogram, one lane
@@ -344,7 +392,8 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
   __shared__ Found s_found[4];
   __shared__ uint32_t s_token;
   __shared__ uint32_t s_pick[2];
-  __shared__ uint16_t s_tile[kLookupTile];
+  __shared__ uint64_t s_scan[kSelectThreads / 64];
+  __shared__ uint16_t s_keys[kBins];  // the distinct values' keys, descending
 
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
@@ -358,8 +407,12 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
 
   // Argmax partials and flags.
   if (tid < 64) {
-    uint64_t key = a.ws.partial_keys[static_cast<uint64_t>(row) * kCountBlocks + tid];
-    uint32_t flags = a.ws.partial_flags[static_cast<uint64_t>(row) * kCountBlocks + tid];
+    uint64_t key = 0;
+    uint32_t flags = 0;
+    if (tid < kCountParts) {
+      key = a.ws.partial_keys[static_cast<uint64_t>(row) * kCountBlocks + tid];
+      flags = a.ws.partial_flags[static_cast<uint64_t>(row) * kCountBlocks + tid];
+    }
     key = wave_max_u64(key);
     flags = wave_or(flags);
     if (tid == 0) {
@@ -391,9 +444,40 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
       count[kBinsPerThread - 3 - 4 * v] = c.z;
       count[kBinsPerThread - 4 - 4 * v] = c.w;
     }
-    uint32_t mine = 0;
+    // The distinct values, compacted in that order, so that their weights are
+    // spread over the workgroup (a random model's logits fill 64 bins of some
+    // fifty threads and none of the others'; their exponentials and the walks
+    // over them took most of the kernel: 113 -> 53 us for 151,936 ids).
+    uint32_t occupied = 0;
 #pragma unroll
-    for (int q = 0; q < kBinsPerThread; ++q) mine += count[q];
+    for (int q = 0; q < kBinsPerThread; ++q) occupied += count[q] != 0;
+    uint32_t distinct = 0;
+    uint32_t slot = block_exclusive_scan<uint32_t>(occupied, &distinct, s_uscan);
+#pragma unroll
+    for (int q = 0; q < kBinsPerThread; ++q)
+      if (count[q]) s_keys[slot++] = static_cast<uint16_t>(top - q);
+    __syncthreads();
+    const uint32_t share = (distinct + kSelectThreads - 1) / kSelectThreads;  // at most kBinsPerThread
+    const uint32_t first = min(distinct, tid * share), past = min(distinct, first + share);
+    const int batches = static_cast<int>((share + kBatch - 1) / kBatch);
+    Batch held;
+    auto read_counts = [&](int b) {
+#pragma unroll
+      for (int q = 0; q < kBatch; ++q) {
+        const uint32_t at = first + b * kBatch + q;
+        held.key[q] = s_keys[min(at, distinct - 1)];
+        held.count[q] = hist[held.key[q]];
+      }
+#pragma unroll
+      for (int q = 0; q < kBatch; ++q)
+        if (first + b * kBatch + q >= past) held.count[q] = 0;
+    };
+    uint32_t mine = 0;
+    for (int b = 0; b < batches; ++b) {
+      read_counts(b);
+#pragma unroll
+      for (int q = 0; q < kBatch; ++q) mine += held.count[q];
+    }
     uint32_t size = 0;
     const uint32_t before = block_exclusive_scan<uint32_t>(mine, &size, s_uscan);
     const uint32_t kept = (set.top_k && size > set.top_k) ? set.top_k : size;
@@ -404,18 +488,32 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
     double mass = 0.0;
     {
       uint32_t left = kept_left;
+      for (int b = 0; b < batches; ++b) {
+        if (batches > 1) read_counts(b);
 #pragma unroll
-      for (int q = 0; q < kBinsPerThread; ++q) {
-        const uint32_t kq = min(count[q], left);
-        left -= kq;
-        if (kq) {
-          const uint32_t key = top - q;
-          const double w = dl_exp((static_cast<double>(order_value(key)) - z0) / set.temperature);
-          w_row[key] = w;
-          mass = mass + static_cast<double>(kq) * w;
+        for (int q = 0; q < kBatch; ++q) {
+          const uint32_t kq = min(held.count[q], left);
+          left -= kq;
+          held.weight[q] = 0.0;
+          if (kq) {
+            const double w = dl_exp((static_cast<double>(order_value(held.key[q])) - z0) / set.temperature);
+            held.weight[q] = w;
+            w_row[held.key[q]] = w;
+            mass = mass + static_cast<double>(kq) * w;
+          }
         }
       }
     }
+    // A thread's values stay in registers when one batch holds them, else
+    // each walk reads them again (the weights are this thread's own stores).
+    auto batch = [&](int b) -> const Batch& {
+      if (batches > 1) {
+        read_counts(b);
+#pragma unroll
+        for (int q = 0; q < kBatch; ++q) held.weight[q] = w_row[held.key[q]];
+      }
+      return held;
+    };
     double total = 0.0;
     const double prefix = block_exclusive_scan<double>(mass, &total, s_dscan);
 
@@ -424,8 +522,8 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
     const double p = set.top_p;
     const double t_lo = p * total * ((1.0 - g) / (1.0 + g)) * (1.0 - 0x1p-50);
     const double t_hi = p * total * ((1.0 + g) / (1.0 - g)) * (1.0 + 0x1p-50);
-    const Found f0 = walk(count, top, prefix, before, kept_left, w_row, t_lo, false);
-    const Found f1 = walk(count, top, prefix, before, kept_left, w_row, t_hi, false);
+    const Found f0 = walk(batches, batch, prefix, before, kept_left, t_lo, false);
+    const Found f1 = walk(batches, batch, prefix, before, kept_left, t_hi, false);
     const uint32_t c_lo = block_min(f0.k, s_uscan);
     const uint32_t c_hi_found = block_min(f1.k, s_uscan);
     if (f0.k != kNone && f0.k == c_lo) s_found[0] = f0;
@@ -443,8 +541,8 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
     const double g2 = 2.0 * g;
     const double d_lo = u * r_lo / (1.0 + g2) * (1.0 - 0x1p-50);
     const double d_hi = u * r_hi / (1.0 - g2) * (1.0 + 0x1p-50);
-    const Found f2 = walk(count, top, prefix, before, kept_left, w_row, d_lo, false);
-    const Found f3 = walk(count, top, prefix, before, kept_left, w_row, d_hi, true);
+    const Found f2 = walk(batches, batch, prefix, before, kept_left, d_lo, false);
+    const Found f3 = walk(batches, batch, prefix, before, kept_left, d_hi, true);
     const uint32_t s_lo = block_min(f2.k, s_uscan);
     const uint32_t s_hi = block_min(f3.k, s_uscan);
     if (f3.k != kNone && f3.k == s_hi) s_found[3] = f3;
@@ -476,39 +574,51 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
     const uint32_t key = s_pick[0];
     uint32_t wanted = s_pick[1];
 
-    // The wanted-th smallest id holding that value.
-    for (uint32_t base = 0; base < a.n; base += kLookupTile) {
-      const uint32_t len = min(static_cast<uint32_t>(kLookupTile), a.n - base);
-      for (uint32_t i = tid; i < len; i += kSelectThreads) s_tile[i] = x[base + i];
-      __syncthreads();
-      uint32_t mine_hits = 0;
-      const uint32_t first = tid * 16;
+    // The wanted-th smallest id holding that value (either zero for the key
+    // of zero): each wavefront counts its part of the row, the one whose part
+    // holds it then finds it.
+    const uint16_t bits = dl_f32_to_bf16(order_value(key)), other = bits == 0 ? uint16_t(0x8000) : bits;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    constexpr int kWavefronts = kSelectThreads / 64, kAhead = 16;
+    const uint32_t part = (a.n + kWavefronts - 1) / kWavefronts;
+    const uint32_t part_begin = min(a.n, wave * part), part_end = min(a.n, part_begin + part);
+    // f(base, mask) per 64 ids until it returns true; the mask of the matches.
+    auto scan = [&](auto&& f) {
+      for (uint32_t base = part_begin; base < part_end; base += 64 * kAhead) {
+        uint16_t v[kAhead];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const uint32_t i = first + e;
-        if (i < len) {
-          const uint32_t v = s_tile[i];
-          mine_hits += (bf16_is_finite(v) && bf16_order(v) == key) ? 1u : 0u;
+        for (int k = 0; k < kAhead; ++k) v[k] = x[min(base + 64 * k + lane, part_end - 1)];
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+          const uint32_t i = base + 64 * k + lane;
+          const uint64_t mask = __ballot(i < part_end && (v[k] == bits || v[k] == other));
+          if (f(base + 64 * k, mask)) return;
         }
       }
-      uint32_t tile_hits = 0;
-      const uint32_t earlier = block_exclusive_scan<uint32_t>(mine_hits, &tile_hits, s_uscan);
-      if (wanted > earlier && wanted <= earlier + mine_hits) {
-        uint32_t left = wanted - earlier;
-        for (int e = 0; e < 16; ++e) {
-          const uint32_t i = first + e;
-          if (i < len) {
-            const uint32_t v = s_tile[i];
-            if (bf16_is_finite(v) && bf16_order(v) == key && --left == 0) {
-              s_token = base + i;
-              break;
-            }
-          }
+    };
+    uint32_t hits = 0;
+    scan([&](uint32_t, uint64_t mask) {
+      hits += __popcll(mask);
+      return false;
+    });
+    if (lane == 0) s_scan[wave] = hits;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) {
+      const uint32_t earlier = static_cast<uint32_t>(s_scan[w]);
+      wanted = wanted > earlier ? wanted - earlier : 0u;
+      if (wanted == 0) break;  // in an earlier part
+    }
+    if (wanted > 0 && wanted <= hits) {
+      scan([&](uint32_t base, uint64_t mask) {
+        const uint32_t here = __popcll(mask);
+        if (wanted > here) {
+          wanted -= here;
+          return false;
         }
-      }
-      __syncthreads();
-      if (wanted <= tile_hits) break;
-      wanted -= tile_hits;
+        const uint64_t below = mask & ((uint64_t(1) << lane) - 1);
+        if (((mask >> lane) & 1u) && __popcll(below) + 1u == wanted) s_token = base + lane;
+        return true;
+      });
     }
     __syncthreads();
     token = s_token;
@@ -536,10 +646,10 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
   }
   if (categorical) {
     __syncthreads();
-    u32x4* dst = reinterpret_cast<u32x4*>(hist + top - (kBinsPerThread - 1));
+    u32x4* dst = reinterpret_cast<u32x4*>(hist);
     const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int v = 0; v < kBinsPerThread / 4; ++v) dst[v] = zero;
+    for (int v = 0; v < kBinsPerThread / 4; ++v) dst[v * kSelectThreads + tid] = zero;
   }
 }
 
@@ -629,7 +739,7 @@ Workspace carve_workspace(void* base, int rows, uint64_t vocabulary) {
 }
 
 void launch_count(hipStream_t stream, const RowsArgs& args) {
-  hipLaunchKernelGGL(k_sample_count, dim3(args.rows * kCountBlocks), dim3(kCountThreads), 0, stream, args);
+  hipLaunchKernelGGL(k_sample_count, dim3(args.rows * kCountParts), dim3(kCountThreads), 0, stream, args);
 }
 
 void launch_select(hipStream_t stream, const RowsArgs& args) {

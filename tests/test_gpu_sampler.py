@@ -260,3 +260,37 @@ def test_terminal_latch_freezes_result(device, queue, oracle, rows):
     assert s.terminal_address() != 0
     with pytest.raises(Exception):
         s.start(settings, 7, [])
+
+
+@pytest.mark.parametrize("kind,n", [("random", 2), ("random", 15), ("random", 17), ("zeros", 1000), ("every value", 65280),
+                                    ("every value", 9000), ("constant", 1100000), ("two values", 140001)])
+def test_counting_parts_and_compaction(device, queue, oracle, kind, n):
+    """Rows shorter than the counting parts, more ids per part than a 16-bit
+    count holds, every finite value at once (64 distinct values per thread),
+    and few distinct values whose j-th occurrence lies anywhere in the row."""
+    from dolittle_amd.sampling import Settings
+    rng = np.random.default_rng(n)
+    if kind == "every value":
+        every = np.arange(65536, dtype=np.uint32)
+        every = every[(every & 0x7f80) != 0x7f80].astype(np.uint16)
+        bits16 = rng.permutation(every)[:n]
+        temperature = 1e36
+    else:
+        values = {"random": rng.standard_normal(n), "zeros": np.where(rng.random(n) < 0.5, 0.0, -0.0),
+                  "constant": np.full(n, 1.5), "two values": np.where(rng.random(n) < 0.3, 2.0, -1.0)}[kind]
+        bits16 = bf16_bits(oracle, values.astype(np.float32))
+        temperature = 0.8
+    logits = oracle.f32_from_bf16(bits16)
+    s = sampler(device, queue, n)
+    buf = device.allocate(2 * n)
+    queue.write(buf, bits16)
+    draws = oracle.MT19937_64(n)
+    for top_k, top_p in ((0, 0.95), (min(n, 7), 1.0), (0, 1.0)):
+        settings = Settings("categorical", temperature, top_k, top_p)
+        for _ in range(4):
+            draw = draws()
+            status, want = oracle.categorical_bits_exp(logits, 1, temperature, top_k, top_p, draw, True)
+            s.submit(buf, settings, draw)
+            assert s.result() == (want, status), (top_k, top_p)
+    s.submit(buf, Settings("greedy", 1.0, 0, 1.0), 0)
+    assert s.result() == (int(np.argmax(logits)), 0)
