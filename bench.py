@@ -283,10 +283,10 @@ def cpu_baseline(model, plan, context, threads, seconds=10.0):
 # sits at 384 visible keys (the bench's last decode position), the "long" one
 # at 4608 (config 3's last).
 TRAFFIC_KERNELS = (
-    (0, "k_qkv<1, 0, 1>", 8, "short"),
-    (4, "k_residual<16, 1, 1>", 8, "short"),
+    (0, "k_qkv<1>", 8, "short"),
+    (4, "k_residual<16, 1>", 8, "short"),
     (5, "k_gateup<1>", 8, "short"),
-    (6, "k_residual<32, 1, 1>", 8, "short"),
+    (6, "k_residual<32, 1>", 8, "short"),
     (7, "k_lm_head<1>", 4, "short"),
     (8, "k_attn_fused", 8, "short"),
     (10, "k_attn_o", 8, "short"),

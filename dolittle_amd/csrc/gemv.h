@@ -57,8 +57,6 @@ __device__ __forceinline__ void stage_put(float* xs, int I, int b, int i, float 
 // Stages BF16 rows [b0, b0 + R) of x (width I) into the P-partial layout.
 // Each thread moves 16-byte chunks; all of a thread's loads are issued
 // before any is consumed.  Requires I % 8 == 0 and I <= 8 * 8 * blockDim.x.
-// `row_stride` (default I) is the distance between source rows, so a block
-// of columns of wider rows can be staged.
 //
 // `active`, when given, is the token loop's grid-uniform liveness word: it
 // is loaded first, and once the row's and the caller's loads are issued a
@@ -67,15 +65,12 @@ __device__ __forceinline__ void stage_put(float* xs, int I, int b, int i, float 
 // after the vector loads are in flight, so a live step waits no longer.
 template <int P, class Issue>
 __device__ __forceinline__ bool stage_rows(const uint16_t* __restrict__ x, int I, int rows, float* xs,
-                                           Issue&& issue, int row_stride = 0, const uint32_t* active = nullptr,
-                                           int valid = 1 << 30) {
+                                           Issue&& issue, const uint32_t* active = nullptr) {
   constexpr int kMaxChunks = 8;
   const int chunks = I / 8;
-  const uint64_t stride = row_stride ? row_stride : I;
   const uint32_t live = active ? *active : 1u;
   for (int b = 0; b < rows; ++b) {
-    // Rows from `valid` on do not exist: their slots repeat the last row.
-    const u32x4* src = reinterpret_cast<const u32x4*>(x + static_cast<uint64_t>(b < valid ? b : valid - 1) * stride);
+    const u32x4* src = reinterpret_cast<const u32x4*>(x + static_cast<uint64_t>(b) * I);
     u32x4 v[kMaxChunks];
 #pragma unroll
     for (int j = 0; j < kMaxChunks; ++j) {
@@ -107,44 +102,6 @@ __device__ __forceinline__ bool stage_rows(const uint16_t* __restrict__ x, int I
     }
   }
   return true;
-}
-
-// Stages the columns [0, I) of B BF16 rows (source rows `row_stride` apart)
-// into the P-partial layout with a compile-time shape: each of the T
-// threads moves I / (8 T) 16-byte chunks per row, all B rows' loads issued
-// before any is converted.  `issue` runs after the loads (loads retire in
-// order).  Requires I % (8 T) == 0.  Only the first `rows` rows exist: the
-// others' slots are staged from the last of them and never stored from.
-template <int P, int B, int I, int T, class Issue>
-__device__ __forceinline__ void stage_block(const uint16_t* __restrict__ x, uint64_t row_stride, float* xs,
-                                            Issue&& issue, int rows = B) {
-  constexpr int J = I / (8 * T);
-  static_assert(J >= 1 && I % (8 * T) == 0, "block width must be a multiple of 8 per thread");
-  u32x4 v[B][J];
-#pragma unroll
-  for (int b = 0; b < B; ++b) {
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-      v[b][j] = reinterpret_cast<const u32x4*>(x + (b < rows ? b : rows - 1) * row_stride)[threadIdx.x + j * T];
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  issue();
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int b = 0; b < B; ++b) {
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int i = (threadIdx.x + j * T) * 8;
-      stage_put<P>(xs, I, b, i + 0, dl_bf16_lo(v[b][j].x));
-      stage_put<P>(xs, I, b, i + 1, dl_bf16_hi(v[b][j].x));
-      stage_put<P>(xs, I, b, i + 2, dl_bf16_lo(v[b][j].y));
-      stage_put<P>(xs, I, b, i + 3, dl_bf16_hi(v[b][j].y));
-      stage_put<P>(xs, I, b, i + 4, dl_bf16_lo(v[b][j].z));
-      stage_put<P>(xs, I, b, i + 5, dl_bf16_hi(v[b][j].z));
-      stage_put<P>(xs, I, b, i + 6, dl_bf16_lo(v[b][j].w));
-      stage_put<P>(xs, I, b, i + 7, dl_bf16_hi(v[b][j].w));
-    }
-  }
 }
 
 // One wavefront computes RW output rows for B input rows.  `tile` points at
@@ -340,10 +297,9 @@ __device__ __forceinline__ float block_rms_inverse(const uint16_t* __restrict__ 
   return inverse;
 }
 
-// Stages round(round(h_b * inverse_b) * gain) for the rows [b0, b0 + R G)
-// that exist (below B) of width D = 128 * kNormK into the staged LDS layouts
-// for P = 16 (when S16) and P = 32 (when S32), computing inverse_b with the
-// reference tree (normalization.cu:134-186) in the same pass.  Thread group
+// to.put(b, i, v) with v = round(round(h_b * inverse_b) * gain) for the rows
+// [b0, b0 + R G) that exist (below B) of width D = 128 * kNormK, computing
+// inverse_b with the reference tree (normalization.cu:134-186) in the same pass.  Thread group
 // g (threads 128 g .. 128 g + 127) owns rows b0 + R g .. b0 + R g + R - 1:
 // thread t of the group keeps features t + 128k of its rows in registers, sums
 // their squares in ascending k (component t), combines groups of four left
@@ -354,10 +310,10 @@ __device__ __forceinline__ float block_rms_inverse(const uint16_t* __restrict__ 
 constexpr int kNormK = 32;
 constexpr int kNormWidth = 128 * kNormK;
 
-template <int R, bool S16, bool S32, int G, class Issue>
-__device__ __forceinline__ bool norm_stage_pass(const uint16_t* __restrict__ h, const uint16_t* __restrict__ gain,
-                                                float eps, float* xs16, float* xs32, float* scratch, int b0, int B,
-                                                Issue&& issue, const uint32_t* active) {
+template <int R, class To, int G, class Issue>
+__device__ __forceinline__ bool norm_rows_pass(const uint16_t* __restrict__ h, const uint16_t* __restrict__ gain,
+                                               float eps, const To& to, float* scratch, int b0, int B, Issue&& issue,
+                                               const uint32_t* active) {
   constexpr int D = kNormWidth;
   const uint32_t live = active ? *active : 1u;
   const int tid = threadIdx.x, t = tid % 128, g = tid / 128;
@@ -409,37 +365,54 @@ __device__ __forceinline__ bool norm_stage_pass(const uint16_t* __restrict__ h, 
       for (int k = 0; k < kNormK; ++k) {
         const float n = dl_round_bf16(dl_round_bf16(hv[b][k] * inverse) * gv[k]);
         const int col = t + 128 * k;
-        if constexpr (S16) stage_put<16>(xs16, D, r0 + b, col, n);
-        if constexpr (S32) stage_put<32>(xs32, D, r0 + b, col, n);
+        to.put(r0 + b, col, n);
       }
     }
   }
   return true;
 }
 
-// norm_stage_pass over B rows, R G at a time (R = 1 row per group while the
+// norm_rows_pass over B rows, R G at a time (R = 1 row per group while the
 // G groups cover the B rows in one pass, else 2) (scratch is reused between
 // passes behind a barrier); G = threads / 128 of the calling workgroup.
-// Rows have width kNormWidth.  Returns false, before any math, when the
-// loop word `active` (read in the first pass, as in stage_rows) is zero.
-// Only the first `rows` (at most B) rows exist and are read and staged; the
-// staged slots of the others are left as they are.
-template <int B, bool S16, bool S32, int G, class Issue>
-__device__ __forceinline__ bool norm_stage(const uint16_t* __restrict__ h, const uint16_t* __restrict__ gain,
-                                           float eps, float* xs16, float* xs32, float* scratch, Issue&& issue,
-                                           const uint32_t* active = nullptr, int rows = B) {
+// Rows have width kNormWidth; to.put(row, column, value) stores each
+// normalized value.  Returns false, before any math, when the loop word `active` (read in
+// the first pass, as in stage_rows) is zero.  Only the first `rows` (at most
+// B) rows exist and are read and stored.
+template <int B, int G, class To, class Issue>
+__device__ __forceinline__ bool norm_rows(const uint16_t* __restrict__ h, const uint16_t* __restrict__ gain, float eps,
+                                          const To& to, float* scratch, Issue&& issue, const uint32_t* active,
+                                          int rows) {
   constexpr int R = B <= G ? 1 : 2;
   auto none = [] {};
 #pragma unroll
   for (int b0 = 0; b0 < B; b0 += R * G) {
     if (b0) {
       __syncthreads();
-      norm_stage_pass<R, S16, S32, G>(h, gain, eps, xs16, xs32, scratch, b0, rows, none, nullptr);
-    } else if (!norm_stage_pass<R, S16, S32, G>(h, gain, eps, xs16, xs32, scratch, b0, rows, issue, active)) {
+      norm_rows_pass<R, To, G>(h, gain, eps, to, scratch, b0, rows, none, nullptr);
+    } else if (!norm_rows_pass<R, To, G>(h, gain, eps, to, scratch, b0, rows, issue, active)) {
       return false;
     }
   }
   return true;
+}
+
+// norm_rows into the staged FP32 layouts for P = 16 (when S16) and P = 32
+// (when S32).
+template <bool S16, bool S32>
+struct StagedFloats {
+  float *xs16, *xs32;
+  __device__ __forceinline__ void put(int b, int col, float v) const {
+    if constexpr (S16) stage_put<16>(xs16, kNormWidth, b, col, v);
+    if constexpr (S32) stage_put<32>(xs32, kNormWidth, b, col, v);
+  }
+};
+
+template <int B, bool S16, bool S32, int G, class Issue>
+__device__ __forceinline__ bool norm_stage(const uint16_t* __restrict__ h, const uint16_t* __restrict__ gain,
+                                           float eps, float* xs16, float* xs32, float* scratch, Issue&& issue,
+                                           const uint32_t* active = nullptr) {
+  return norm_rows<B, G>(h, gain, eps, StagedFloats<S16, S32>{xs16, xs32}, scratch, issue, active, B);
 }
 
 }  // namespace dl

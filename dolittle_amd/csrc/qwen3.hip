@@ -43,6 +43,7 @@
 #include "heads.h"
 #include "nla.h"
 #include "prefill.h"
+#include "rows_mfma.h"
 #include "sampler.h"
 
 namespace dl {
@@ -52,11 +53,6 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kBlock = kWaves * 64;
-// Wavefronts per workgroup of the GEMV kernels for `rows` staged rows.  From
-// four rows the staged inputs fill most of the LDS, so one workgroup is
-// resident per CU; eight wavefronts (two per SIMD) keep twice the weight
-// loads in flight.
-constexpr int gemv_waves(int rows) { return rows >= 4 ? 8 : kWaves; }
 constexpr int kHeadDim = 128;
 
 __device__ __forceinline__ uint16_t bf16_bits(float v) { return dl_f32_to_bf16(v); }
@@ -309,48 +305,22 @@ struct QkvArgs {
   uint64_t cache_seq_stride; // elements
   int D, QW, KW, cap;
   float eps;
-  // Rows of the launch that exist (a launch of a larger row template for
-  // fewer rows reads and writes only these; see live_rows).
-  int rows = 1 << 30;
+  int rows;  // rows that exist (k_rows_qkv: at most its row template)
 };
 
-// Rows that exist in a launch of the B-row kernels given the launch's `rows`
-// field.  Only the 4- and 8-row kernels run for fewer rows (the host takes
-// one or two rows with kernels of that size), so for B <= 2 this is B and
-// the row guards compile away.
-template <int B>
-__device__ __forceinline__ int live_rows(int rows) {
-  if constexpr (B <= 2) {
-    return B;
-  } else {
-    return rows < B ? rows : B;
-  }
-}
-
-// Part: kQkvAll projects Q, K and V; at eight rows both staged layouts do
-// not fit in LDS together, so kQkvQ (Q rows, P = 16 layout) and kQkvKV (K
-// and V rows, P = 32 layout) run in separate workgroups (k_qkv_roles).
-enum QkvPart : int { kQkvAll = 0, kQkvQ = 1, kQkvKV = 2 };
 // Input width of the batch-1 GEMV paths that hold a wavefront's whole weight
 // tile in registers (Qwen3-8B's hidden width).
 constexpr int kWholeTileInputs = 4096;
-constexpr int qkv_waves(int rows, int part) { return part == kQkvAll ? kWaves : gemv_waves(rows); }
 
-// Split > 1 divides each tile's B rows into Split work items of B / Split
-// rows (the same tile's weights, read by Split wavefronts): with one tile
-// per wavefront the chain length per wavefront, not the CU count, bounds
-// these launches at eight rows.
-// `block` of `blocks` is the workgroup's place among the launch's
-// workgroups of this part (k_qkv_roles runs the Q and K/V parts of eight
-// rows in one launch).
-template <int B, int Part, int Split>
-__device__ __forceinline__ void qkv_rows(const QkvArgs& a, int block, int blocks) {
-  constexpr int W = qkv_waves(B, Part);
-  constexpr int BR = B / Split;
-  static_assert(B % Split == 0, "rows split evenly");
+// Two wavefronts per SIMD at least: the batch-1 whole-tile path holds 128
+// weight VGPRs, and a grid of one tile per wavefront must be resident at once.
+template <int B>
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void k_qkv(QkvArgs a) {
+  static_assert(B <= 2, "more rows run k_rows_qkv");
+  constexpr int W = kWaves;
   extern __shared__ float lds[];
   float* xs16 = lds;
-  float* xs32 = Part == kQkvKV ? lds : xs16 + B * staged_floats(16, a.D);
+  float* xs32 = xs16 + B * staged_floats(16, a.D);
   __shared__ float scratch[W * 40];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int q_tiles = a.QW / 4, k_tiles = a.KW / 2, total = q_tiles + 2 * k_tiles;
@@ -365,17 +335,15 @@ __device__ __forceinline__ void qkv_rows(const QkvArgs& a, int block, int blocks
     if (is_v) kt -= k_tiles;
     return a.w + q_tiles * q_chunks + (is_v ? k_tiles : 0) * k_chunks + kt * k_chunks;
   };
-  const int tile_begin = Part == kQkvKV ? q_tiles : 0, tile_end = Part == kQkvQ ? q_tiles : total;
-  const int items = (tile_end - tile_begin) * Split;
-  const int first = block * W + wave;
-  if constexpr (B == 1 && Part == kQkvAll && Split == 1) {
-    if (blocks * W >= items && a.D == kWholeTileInputs) {
+  const int first = blockIdx.x * W + wave;
+  if constexpr (B == 1) {
+    if (static_cast<int>(gridDim.x) * W >= total && a.D == kWholeTileInputs) {
       // One tile per wavefront, held in registers (32 chunks per lane for a
       // Q tile, 16 for K or V): the first 16 chunks are issued before the
       // prologue, the rest right after it, and the chains run from
       // registers; the same chain steps as chain_tile.
-      const bool has = first < items;
-      const int tile = tile_begin + first;
+      const int tile = first;
+      const bool has = tile < total;
       const bool is_q = tile < q_tiles;
       constexpr int SQ = kWholeTileInputs / 128, SK = kWholeTileInputs / 256;
       u32x4 w[SQ];
@@ -428,70 +396,45 @@ __device__ __forceinline__ void qkv_rows(const QkvArgs& a, int block, int blocks
   FirstBatch fb{};
   // The prologue returns, after issuing its loads, when the loop is stopped
   // (grid-uniform flag).
-  const int rows = live_rows<B>(a.rows);
-  if (!norm_stage<B, Part != kQkvKV, Part != kQkvQ, W / 2>(
+  if (!norm_stage<B, true, true, W / 2>(
           a.h, a.norm, a.eps, xs16, xs32, scratch,
           [&] {
-            if (first < items) issue_first(tile_src(tile_begin + first / Split), lane, fb);
+            if (first < total) issue_first(tile_src(first), lane, fb);
           },
-          &a.ctl->active, rows))
+          &a.ctl->active))
     return;
   __syncthreads();
   const uint64_t pos = a.ctl->position;
-  for (int item = first; item < items; item += blocks * W) {
-    const int tile = tile_begin + item / Split, b0 = (item % Split) * BR;
+  for (int tile = first; tile < total; tile += gridDim.x * W) {
     const bool is_q = tile < q_tiles;
     int kt = tile - q_tiles;
     const bool is_v = !is_q && kt >= k_tiles;
     if (is_v) kt -= k_tiles;
     const u32x4* src = tile_src(tile);
-    const int next = item + blocks * W;
-    const u32x4* next_src = next < items ? tile_src(tile_begin + next / Split) : nullptr;
-    float acc[BR];
-    if (Part == kQkvQ || (Part == kQkvAll && is_q)) {
-      chain_tile<16, BR>(src, xs16 + b0 * staged_floats(16, a.D), a.D, lane, acc, &fb, next_src);
+    const int next = tile + gridDim.x * W;
+    const u32x4* next_src = next < total ? tile_src(next) : nullptr;
+    float acc[B];
+    if (is_q) {
+      chain_tile<16, B>(src, xs16, a.D, lane, acc, &fb, next_src);
       if (lane % 16 == 0) {
         const int row = tile * 4 + lane / 16;
 #pragma unroll
-        for (int b = 0; b < BR; ++b)
-          if (b0 + b < rows) a.q_out[(b0 + b) * a.QW + row] = bf16_bits(acc[b]);
+        for (int b = 0; b < B; ++b) a.q_out[b * a.QW + row] = bf16_bits(acc[b]);
       }
     } else {
-      chain_tile<32, BR>(src, xs32 + b0 * staged_floats(32, a.D), a.D, lane, acc, &fb, next_src);
+      chain_tile<32, B>(src, xs32, a.D, lane, acc, &fb, next_src);
       if (lane % 32 == 0) {
         const int row = kt * 2 + lane / 32;
 #pragma unroll
-        for (int b = 0; b < BR; ++b) {
-          if (b0 + b >= rows) break;
+        for (int b = 0; b < B; ++b) {
           if (is_v)
-            a.v_cache[(b0 + b) * a.cache_seq_stride + static_cast<uint64_t>(row) * a.cap + pos] = bf16_bits(acc[b]);
+            a.v_cache[b * a.cache_seq_stride + static_cast<uint64_t>(row) * a.cap + pos] = bf16_bits(acc[b]);
           else
-            a.k_out[(b0 + b) * a.KW + row] = bf16_bits(acc[b]);
+            a.k_out[b * a.KW + row] = bf16_bits(acc[b]);
         }
       }
     }
   }
-}
-
-// Two wavefronts per SIMD at least: the batch-1 whole-tile path holds 128
-// weight VGPRs, and a grid of one tile per wavefront must be resident at once.
-template <int B, int Part = kQkvAll, int Split = 1>
-__global__ __launch_bounds__(qkv_waves(B, Part) * 64) __attribute__((amdgpu_waves_per_eu(2))) void k_qkv(QkvArgs a) {
-  qkv_rows<B, Part, Split>(a, blockIdx.x, gridDim.x);
-}
-
-// The Q part (workgroups [0, q_blocks)) and the K/V part (the rest) of B
-// rows in one launch: a compute unit whose Q workgroup is done takes a K/V
-// workgroup without waiting for the whole Q grid.  Each workgroup stages only
-// its part's layout, so both fit the LDS that one of them takes.
-template <int B, int Split>
-__global__ __launch_bounds__(qkv_waves(B, kQkvQ) * 64) __attribute__((amdgpu_waves_per_eu(2))) void k_qkv_roles(
-    QkvArgs a, int q_blocks) {
-  static_assert(qkv_waves(B, kQkvQ) == qkv_waves(B, kQkvKV), "both parts use the same workgroup shape");
-  if (static_cast<int>(blockIdx.x) < q_blocks)
-    qkv_rows<B, kQkvQ, Split>(a, blockIdx.x, q_blocks);
-  else
-    qkv_rows<B, kQkvKV, Split>(a, blockIdx.x - q_blocks, gridDim.x - q_blocks);
 }
 
 // Orders one wavefront's LDS writes before its own later LDS reads (and the
@@ -522,10 +465,16 @@ struct AttnArgs {
   // sequences at one position (decode), 1 when they are consecutive
   // positions of one sequence (cache_seq_stride 0, chunked prompt pass).
   int pos_step;
-  // The output rows in P16 order, for the many-row exact O projection (the
-  // row-block kernels only).
+  // The output rows in P16 order, which the O projections of three rows and
+  // more read (no kernel that hands the rows over inside its launch).
   int permuted_out;
 };
+
+// Place of feature `f` of an output row.
+__device__ __forceinline__ int att_place(const AttnArgs& a, int f) {
+  return a.permuted_out ? static_cast<int>(prefill::permuted(static_cast<uint32_t>(f), 16)) : f;
+}
+
 
 
 // Grid (kv head, 64-key tile, sequence); block 256 = 4 waves, one per query
@@ -1276,8 +1225,8 @@ __global__ __launch_bounds__(kPwThreads) void k_attn_pv_rows(AttnArgs a) {
   if (wave == 2) second[lane] = acc;
   __syncthreads();
   if (wave == 0)
-    a.att[static_cast<uint64_t>(b) * a.q_heads * kHeadDim + (g * group + hl) * kHeadDim + fb * kPwFeatures + f] =
-        bf16_bits(acc + second[lane]);
+    a.att[static_cast<uint64_t>(b) * a.q_heads * kHeadDim + (g * group + hl) * kHeadDim +
+          att_place(a, fb * kPwFeatures + f)] = bf16_bits(acc + second[lane]);
 }
 
 // k_attn_pv_rows for the rows of the chunked prompt pass (consecutive
@@ -1498,8 +1447,7 @@ __global__ __launch_bounds__(kPwThreads) void k_attn_pv_block(AttnArgs a, int ro
 #pragma unroll
         for (int i = 0; i < kPbFeat; ++i)
           a.att[static_cast<uint64_t>(rb + rr) * a.q_heads * kHeadDim + (g * group + hl) * kHeadDim +
-                (a.permuted_out ? static_cast<int>(prefill::permuted(f0 + i, 16)) : f0 + i)] =
-              bf16_bits(acc[rr][i] + second[rr][i][lane]);
+                att_place(a, f0 + i)] = bf16_bits(acc[rr][i] + second[rr][i][lane]);
       }
   }
 }
@@ -1971,7 +1919,8 @@ __device__ __forceinline__ bool attn_fused_body(const AttnArgs& a, int slot, int
       __builtin_amdgcn_s_waitcnt(pv_vmcnt(0));
     }
   } else {
-    if (tid < kPartFeatures) att[tid] = bf16_bits(red[tid] + red[tid + kHeadDim]);
+    if (tid < kPartFeatures)
+      (att - part * kPartFeatures)[att_place(a, part * kPartFeatures + tid)] = bf16_bits(red[tid] + red[tid + kHeadDim]);
   }
   return true;
 }
@@ -1995,9 +1944,7 @@ struct ResidualArgs {
   // with same_sequence, consecutive positions of sequence `sequence`
   // (row r at ctl->position + r; chunked prompt pass).
   int same_sequence, sequence;
-  // Rows from row0 that exist (a launch of a larger row template for fewer
-  // rows reads and writes only these).
-  int rows = 1 << 30;
+  int rows;  // rows from row0 that exist (see QkvArgs::rows)
 };
 
 
@@ -2038,25 +1985,22 @@ __device__ __forceinline__ void residual_outputs(const ResidualArgs& a, const fl
       for (int b = 0; b < B; ++b) ep[(lane / P) * B + b] = acc[b];
     }
     wave_lds_sync();
-    if (lane < RW * B && lane % B < live_rows<B>(a.rows)) finish(lane / B, lane % B, ep[lane]);
+    if (lane < RW * B) finish(lane / B, lane % B, ep[lane]);
     wave_lds_sync();
   }
 }
 
 // y = round(x W^T); h = round(h + y); optionally h = round(h + steer) and a
 // copy of h into the capture arena at the current position.
-// Split as in k_qkv: each tile's rows as Split work items of B / Split rows.
-template <int P, int B, int Split = 1>
-__global__ __launch_bounds__(gemv_waves(B) * 64) void k_residual(ResidualArgs a) {
-  constexpr int W = gemv_waves(B);
-  constexpr int BR = B / Split;
-  static_assert(B % Split == 0, "rows split evenly");
+template <int P, int B>
+__global__ __launch_bounds__(kWaves * 64) void k_residual(ResidualArgs a) {
+  constexpr int W = kWaves;
+  static_assert(B <= 2, "more rows run k_rows_o and k_rows_down");
   extern __shared__ float xs[];
-  __shared__ float epi[W * (64 / P) * BR];
+  __shared__ float epi[W * (64 / P) * B];
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   constexpr int RW = 64 / P;
   const int tiles = a.D / RW;
-  const int items = tiles * Split;
   const int S = a.I / (8 * P);
   const uint64_t chunks = static_cast<uint64_t>(S) * 64;
   const int first = blockIdx.x * W + wave;
@@ -2066,85 +2010,22 @@ __global__ __launch_bounds__(gemv_waves(B) * 64) void k_residual(ResidualArgs a)
   if (!stage_rows<P>(
           a.x + static_cast<uint64_t>(a.row0) * a.I, a.I, B, xs,
           [&] {
-            if (first < items) issue_first(a.w + (first / Split) * chunks, lane, fb);
+            if (first < tiles) issue_first(a.w + first * chunks, lane, fb);
           },
-          0, &a.ctl->active, live_rows<B>(a.rows)))
+          &a.ctl->active))
     return;
   __syncthreads();
   const uint64_t pos = a.ctl->position;
   const bool steer = a.steer != nullptr && a.layer == a.ctl->steer_layer;
   const bool capture = a.capture != nullptr && a.layer == a.ctl->capture_layer;
   const uint32_t steer_mask = a.ctl->steer_mask;
-  for (int item = first; item < items; item += gridDim.x * W) {
-    const int tile = item / Split, b0 = (item % Split) * BR;
-    float acc[BR];
-    const int next = item + gridDim.x * W;
+  for (int tile = first; tile < tiles; tile += gridDim.x * W) {
+    float acc[B];
+    const int next = tile + gridDim.x * W;
     // One tile per wavefront at B = 1 leaves one or two wavefronts per SIMD:
     // two batches in flight per wavefront keep more of HBM busy.
-    chain_tile<P, BR, true>(a.w + tile * chunks, xs + b0 * staged_floats(P, a.I), a.I, lane, acc, &fb,
-                            next < items ? a.w + (next / Split) * chunks : nullptr);
-    if constexpr (Split == 1) {
-      residual_outputs<P, BR>(a, acc, tile, lane, epi + wave * RW * BR, pos, steer, capture, steer_mask);
-    } else {
-      ResidualArgs part = a;
-      part.row0 += b0;
-      part.rows -= b0;
-      residual_outputs<P, BR>(part, acc, tile, lane, epi + wave * RW * BR, pos, steer, capture, steer_mask);
-    }
-  }
-}
-
-// k_residual for rows whose staged inputs do not fit in LDS at once (the
-// down projection, I = 12288, at four or more rows): the inputs are staged
-// kChunkInputs at a time and every wavefront carries its chains across the
-// blocks in ascending input order, so each partial is the same FMA chain as
-// in k_residual.  Each wavefront owns one tile per pass; all wavefronts of a
-// workgroup take part in every staging barrier (uniform trip counts).
-constexpr int kChunkInputs = 4096;
-
-template <int P, int B>
-__global__ __launch_bounds__(gemv_waves(B) * 64) void k_residual_chunked(ResidualArgs a) {
-  constexpr int W = gemv_waves(B);
-  constexpr int kChunkSteps = kChunkInputs / (8 * P);
-  extern __shared__ float xs[];
-  __shared__ float epi[W * (64 / P) * B];
-  if (!a.ctl->active) return;
-  const uint64_t pos = a.ctl->position;
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  constexpr int RW = 64 / P;
-  const int tiles = a.D / RW;
-  const int S = a.I / (8 * P);
-  const uint64_t chunks = static_cast<uint64_t>(S) * 64;
-  const int blocks = a.I / kChunkInputs;
-  const bool steer = a.steer != nullptr && a.layer == a.ctl->steer_layer;
-  const bool capture = a.capture != nullptr && a.layer == a.ctl->capture_layer;
-  const uint32_t steer_mask = a.ctl->steer_mask;
-  for (int base = blockIdx.x * W; base < tiles; base += gridDim.x * W) {
-    const int tile = base + wave;
-    const bool active = tile < tiles;
-    const u32x4* src = a.w + static_cast<uint64_t>(active ? tile : base) * chunks;
-    float acc[B];
-#pragma unroll
-    for (int b = 0; b < B; ++b) acc[b] = 0.0f;
-    FirstBatch fb{};
-    for (int c = 0; c < blocks; ++c) {
-      __syncthreads();  // every wavefront is done with the previous block
-      stage_block<P, B, kChunkInputs, W * 64>(a.x + static_cast<uint64_t>(a.row0) * a.I + c * kChunkInputs, a.I, xs,
-                                             [&] {
-                                               if (c == 0 && active) issue_first(src, lane, fb);
-                                             },
-                                             live_rows<B>(a.rows));
-      __syncthreads();
-      if (active) {
-        // The block width is passed as a run-time value (a.I / blocks): a
-        // compile-time width lets the compiler unroll the whole block and
-        // hoist its LDS reads past the register file.
-        const u32x4* at = src + static_cast<uint64_t>(c) * kChunkSteps * 64;
-        chain_body<P, B>(at, xs, a.I / blocks, lane, acc, &fb, c + 1 < blocks ? at + kChunkSteps * 64 : nullptr);
-      }
-    }
-    chain_merge<P, B>(acc);
-    if (active) residual_outputs<P, B>(a, acc, tile, lane, epi + wave * RW * B, pos, steer, capture, steer_mask);
+    chain_tile<P, B, true>(a.w + tile * chunks, xs, a.I, lane, acc, &fb, next < tiles ? a.w + next * chunks : nullptr);
+    residual_outputs<P, B>(a, acc, tile, lane, epi + wave * RW * B, pos, steer, capture, steer_mask);
   }
 }
 
@@ -2419,12 +2300,12 @@ struct GateUpArgs {
   uint16_t* act;         // [B][F]
   int D, F;
   float eps;
-  int rows = 1 << 30;    // rows that exist (see QkvArgs::rows)
+  int rows;              // rows that exist (see QkvArgs::rows)
 };
 
 template <int B>
-__global__ __launch_bounds__(gemv_waves(B) * 64) void k_gateup(GateUpArgs a) {
-  constexpr int W = gemv_waves(B);
+__global__ __launch_bounds__(kWaves * 64) void k_gateup(GateUpArgs a) {
+  constexpr int W = kWaves;
   extern __shared__ float xs[];
   __shared__ float scratch[W * 40];
   __shared__ float epi[W * 4 * B];
@@ -2441,7 +2322,7 @@ __global__ __launch_bounds__(gemv_waves(B) * 64) void k_gateup(GateUpArgs a) {
           [&] {
             if (first < tiles) issue_first(a.w + first * chunks, lane, fb);
           },
-          &a.ctl->active, live_rows<B>(a.rows)))
+          &a.ctl->active))
     return;
   __syncthreads();
   (void)S;
@@ -2463,7 +2344,7 @@ __global__ __launch_bounds__(gemv_waves(B) * 64) void k_gateup(GateUpArgs a) {
         for (int b = 0; b < B; ++b) ep[(lane / 16) * B + b] = acc[b];
       }
       wave_lds_sync();
-      if (lane < 2 * B && lane % B < live_rows<B>(a.rows)) {
+      if (lane < 2 * B) {
         const int o = lane / B, b = lane % B;
         a.act[static_cast<uint64_t>(b) * a.F + tile * 2 + o] =
             bf16_bits(silu_times(rbf(ep[o * B + b]), rbf(ep[(2 + o) * B + b])));
@@ -2591,7 +2472,7 @@ struct HeadArgs {
   uint32_t V;
   float eps;
   int row0;                // first sequence of this launch's row group
-  int rows = 1 << 30;      // rows from row0 that exist (see QkvArgs::rows)
+  int rows;                // rows from row0 that exist (see QkvArgs::rows)
 };
 
 // Orders BF16 logits: key = (ordered value << 32) | ~id, so the maximum key
@@ -2623,8 +2504,8 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
 }
 
 template <int B>
-__global__ __launch_bounds__(gemv_waves(B) * 64) void k_lm_head(HeadArgs a) {
-  constexpr int W = gemv_waves(B);
+__global__ __launch_bounds__(kWaves * 64) void k_lm_head(HeadArgs a) {
+  constexpr int W = kWaves;
   extern __shared__ float xs[];
   __shared__ float scratch[W * 40];
   __shared__ uint64_t wave_keys[W][B];
@@ -2637,11 +2518,10 @@ __global__ __launch_bounds__(gemv_waves(B) * 64) void k_lm_head(HeadArgs a) {
   const int first = blockIdx.x * W + wave;
   (void)S;
   FirstBatch fb{};
-  const int rows = live_rows<B>(a.rows);
   norm_stage<B, true, false, W / 2>(a.h + static_cast<uint64_t>(a.row0) * a.D, a.norm, a.eps, xs, nullptr, scratch,
                                     [&] {
     if (first < tiles) issue_first(a.w + first * chunks, lane, fb);
-  }, nullptr, rows);
+  });
   __syncthreads();
   uint64_t best[B];
   uint32_t flags[B];
@@ -2658,7 +2538,6 @@ __global__ __launch_bounds__(gemv_waves(B) * 64) void k_lm_head(HeadArgs a) {
       const uint32_t row = static_cast<uint32_t>(tile * 4 + lane / 16);
 #pragma unroll
       for (int b = 0; b < B; ++b) {
-        if (b >= rows) break;
         const uint16_t bits = bf16_bits(acc[b]);
         a.logits[static_cast<uint64_t>(a.row0 + b) * a.V + row] = bits;
         logit_key(bits, row, &best[b], &flags[b]);
@@ -2677,7 +2556,7 @@ __global__ __launch_bounds__(gemv_waves(B) * 64) void k_lm_head(HeadArgs a) {
     }
   }
   __syncthreads();
-  if (static_cast<int>(threadIdx.x) < rows) {
+  if (threadIdx.x < B) {
     const int b = threadIdx.x;
     uint64_t k = 0;
     uint32_t f = 0;
@@ -2687,6 +2566,354 @@ __global__ __launch_bounds__(gemv_waves(B) * 64) void k_lm_head(HeadArgs a) {
     }
     a.partial_keys[static_cast<uint64_t>(a.row0 + b) * gridDim.x + blockIdx.x] = k;
     a.partial_flags[static_cast<uint64_t>(a.row0 + b) * gridDim.x + blockIdx.x] = f;
+  }
+}
+
+// ------------------------------------------- GEMVs of three to eight rows
+// The decode kernels' projections for R = 4 or 8 rows (fewer may exist) on
+// depth-1 FP32 MFMA (rows_mfma.h); the same chains, merges and rounding points.
+//
+// Bound: the weight stream (a compute unit takes about 25 bytes per ns), after
+// the launch and the norm prologue: the 201 MB gate/up launch is 29 us of HBM
+// at its streaming rate, about 8 us of a tile per wavefront and 10 before the
+// first.  Qwen3-8B block at 8 rows against the vector-ALU form (an FMA per row
+// and element, the inputs as FP32 in LDS): gate/up 44.8 -> 42.4 us, down 30.5
+// -> 27.6, QKV 21.6 -> 19.3, O 14.9 -> 11.4, LM head 262-277 -> 215-231; at 4
+// rows O 12.1 -> 9.5 and the others equal (within 1 us).  One workgroup of
+// eight wavefronts per compute unit (four for O, one tile each); measured for
+// gate/up at 8 rows: 12 or 16 wavefronts 45 and 56 us, two workgroups per
+// compute unit 58, two or three tiles at a time in one wavefront 46-56, a
+// whole tile held in registers 47-50.
+constexpr int kRowWaves = 8;
+
+template <int R>
+struct RowStage {
+  static constexpr int G = R / 4;
+  static constexpr int kChunks = kNormWidth / 128;  // chunks of one 4096-wide row, or of one block of wider ones
+  static constexpr int kPieces = G * kChunks;
+  static constexpr int kGroup = kChunks * 64;       // slots between row groups
+  static constexpr int kBytes = kPieces * 1024;
+};
+
+// Where norm_rows stores its rows: the staged BF16 rows in P16 or P32 order.
+template <int R>
+struct StagedRows {
+  uint16_t* xs;
+  bool p16;
+  __device__ __forceinline__ void put(int row, int col, float v) const {
+    const int at = p16 ? rows::staged_element<16>(row, col, RowStage<R>::kChunks)
+                       : rows::staged_element<32>(row, col, RowStage<R>::kChunks);
+    xs[at] = static_cast<uint16_t>(__float_as_uint(v) >> 16);
+  }
+};
+
+// The wavefront's slot in every piece (rows::slot_of for its partial and row).
+__device__ __forceinline__ int row_slot(int lane) { return rows::slot_of(lane / 4, lane % 4); }
+
+__device__ __forceinline__ void zero(rows::f32x4& v) { v = rows::f32x4{0.0f, 0.0f, 0.0f, 0.0f}; }
+
+// Two wavefronts share a P = 32 tile, each with 16 partials (h = 0, 1): offset
+// 16 across them through `exchange` ([pair][G][64]).  Every wavefront of the
+// workgroup calls; true where the sums are (h = 0).
+template <int G>
+__device__ __forceinline__ bool merge_pair(rows::f32x4 (&acc)[G], rows::f32x4* exchange, int wave, int lane) {
+  rows::f32x4* at = exchange + (wave / 2) * G * 64 + lane;
+  __syncthreads();
+  if (wave % 2) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) at[g * 64] = acc[g];
+  }
+  __syncthreads();
+  if (wave % 2) return false;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const rows::f32x4 upper = at[g * 64];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[g][i] = acc[g][i] + upper[i];
+  }
+  return true;
+}
+
+// Workgroups [0, q_blocks) project Q (one tile of four outputs per wavefront
+// at a time), the rest K and V (half the partials of a tile per wavefront).
+template <int R>
+__global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void k_rows_qkv(QkvArgs a,
+                                                                                                     int q_blocks) {
+  using S = RowStage<R>;
+  constexpr int G = S::G;
+  __shared__ __align__(1024) uint8_t xs[S::kBytes];
+  __shared__ rows::f32x4 exchange[kRowWaves / 2 * G * 64];
+  __shared__ float scratch[kRowWaves * 40];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const bool q_part = static_cast<int>(blockIdx.x) < q_blocks;
+  const int rows = min(a.rows, R);
+  const int q_steps = a.D / 128, kv_steps = a.D / 256, q_tiles = a.QW / 4, kv_tiles = 2 * a.KW / 4;
+  const int h = wave % 2;
+  auto q_src = [&](int tile) { return a.w + static_cast<uint64_t>(tile) * q_steps * 64 + rows::lane_chunk16(lane); };
+  auto kv_src = [&](int tile) {
+    return a.w + static_cast<uint64_t>(q_tiles) * q_steps * 64 + static_cast<uint64_t>(tile) * 2 * kv_steps * 64 +
+           rows::lane_chunk32(lane, h, kv_steps);
+  };
+  const int blocks = q_part ? q_blocks : static_cast<int>(gridDim.x) - q_blocks;
+  const int block = q_part ? blockIdx.x : blockIdx.x - q_blocks;
+  const int per_block = q_part ? kRowWaves : kRowWaves / 2;
+  const int tiles = q_part ? q_tiles : kv_tiles;
+  const int first = block * per_block + (q_part ? wave : wave / 2);
+  FirstBatch fb{};
+  auto src = [&](int tile) { return q_part ? q_src(tile) : kv_src(tile); };
+  if (!norm_rows<R, kRowWaves / 2>(
+          a.h, a.norm, a.eps, StagedRows<R>{reinterpret_cast<uint16_t*>(xs), q_part}, scratch,
+          [&] {
+            if (first < tiles) issue_first(src(first), 0, fb);
+          },
+          &a.ctl->active, rows))
+    return;
+  __syncthreads();
+  const uint64_t pos = a.ctl->position;
+  const u32x4* x = reinterpret_cast<const u32x4*>(xs) + row_slot(lane);
+  const int q = lane / 16, b = lane % 16;
+  if (q_part) {
+    for (int tile = first; tile < tiles; tile += blocks * per_block) {
+      rows::f32x4 acc[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) zero(acc[g]);
+      const int next = tile + blocks * per_block;
+      rows::chain<G>(q_src(tile), x, 64, S::kGroup, q_steps, acc, fb, next < tiles ? q_src(next) : nullptr);
+      const float v = rows::merge<G>(acc, lane);
+      if (b < rows) a.q_out[static_cast<uint64_t>(b) * a.QW + tile * 4 + rows::output_of(q)] = bf16_bits(v);
+    }
+    return;
+  }
+  for (int base = block * per_block; base < tiles; base += blocks * per_block) {
+    const int tile = base + wave / 2, next = tile + blocks * per_block;
+    rows::f32x4 acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) zero(acc[g]);
+    if (tile < tiles)
+      rows::chain<G>(kv_src(tile), x + h * 64, 128, S::kGroup, kv_steps, acc, fb, next < tiles ? kv_src(next) : nullptr);
+    if (!merge_pair<G>(acc, exchange, wave, lane) || tile >= tiles) continue;
+    const float v = rows::merge<G>(acc, lane);
+    const int row = tile * 4 + rows::output_of(q);
+    if (b >= rows) continue;
+    if (row < a.KW)
+      a.k_out[static_cast<uint64_t>(b) * a.KW + row] = bf16_bits(v);
+    else
+      a.v_cache[b * a.cache_seq_stride + static_cast<uint64_t>(row - a.KW) * a.cap + pos] = bf16_bits(v);
+  }
+}
+
+// O: the P16-ordered attention rows, one tile of four outputs per wavefront.
+// Queries wider than the staged 4096 inputs have P = 32 and no O kernel here.
+template <int R, int Waves>
+__global__ __launch_bounds__(Waves * 64) void k_rows_o(ResidualArgs a) {
+  using S = RowStage<R>;
+  constexpr int G = S::G;
+  __shared__ __align__(1024) uint8_t xs[S::kBytes];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int rows = min(a.rows, R), steps = a.I / 128, tiles = a.D / 4;
+  const int first = blockIdx.x * Waves + wave;
+  auto src = [&](int tile) { return a.w + static_cast<uint64_t>(tile) * steps * 64 + rows::lane_chunk16(lane); };
+  const uint32_t live = a.ctl->active;
+  rows::stage_permuted<R, S::kChunks, Waves>(a.x + static_cast<uint64_t>(a.row0) * a.I, a.I, 0, steps, rows, xs, wave,
+                                             lane);
+  __builtin_amdgcn_sched_barrier(0);
+  FirstBatch fb{};
+  if (first < tiles) issue_first(src(first), 0, fb);
+  __builtin_amdgcn_sched_barrier(0);
+  if (!live) {
+    __builtin_amdgcn_s_waitcnt(rows::vm_wait(0));  // no load outlives the workgroup
+    return;
+  }
+  if (first < tiles)
+    __builtin_amdgcn_s_waitcnt(rows::vm_wait(kBatch));  // the staged rows, issued before the weights
+  else
+    __builtin_amdgcn_s_waitcnt(rows::vm_wait(0));
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  const uint64_t pos = a.ctl->position;
+  const bool steer = a.steer != nullptr && a.layer == a.ctl->steer_layer;
+  const bool capture = a.capture != nullptr && a.layer == a.ctl->capture_layer;
+  const uint32_t steer_mask = a.ctl->steer_mask;
+  const u32x4* x = reinterpret_cast<const u32x4*>(xs) + row_slot(lane);
+  for (int tile = first; tile < tiles; tile += gridDim.x * Waves) {
+    rows::f32x4 acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) zero(acc[g]);
+    const int next = tile + gridDim.x * Waves;
+    rows::chain<G>(src(tile), x, 64, S::kGroup, steps, acc, fb, next < tiles ? src(next) : nullptr);
+    const float v = rows::merge<G>(acc, lane);
+    if (lane % 16 < rows)
+      residual_store(a, tile * 4 + rows::output_of(lane / 16), lane % 16, v, pos, steer, capture, steer_mask);
+  }
+}
+
+// Down: the P32-ordered activations staged 4096 inputs at a time in two
+// buffers, the next block's loads in flight while the chains run this one.
+template <int R>
+__global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void k_rows_down(ResidualArgs a) {
+  using S = RowStage<R>;
+  constexpr int G = S::G, kSteps = S::kChunks / 2;
+  __shared__ __align__(1024) uint8_t x0[S::kBytes], x1[S::kBytes];
+  __shared__ rows::f32x4 exchange[kRowWaves / 2 * G * 64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int h = wave % 2, rows = min(a.rows, R);
+  const int steps = a.I / 256, chunks = a.I / 128, blocks = (steps + kSteps - 1) / kSteps, tiles = a.D / 4;
+  if (!a.ctl->active) return;
+  const uint64_t pos = a.ctl->position;
+  const bool steer = a.steer != nullptr && a.layer == a.ctl->steer_layer;
+  const bool capture = a.capture != nullptr && a.layer == a.ctl->capture_layer;
+  const uint32_t steer_mask = a.ctl->steer_mask;
+  const uint16_t* xrow = a.x + static_cast<uint64_t>(a.row0) * a.I;
+  const int slot = h * 64 + row_slot(lane);
+  auto stage = [&](int block, uint8_t* xs) {
+    rows::stage_permuted<R, S::kChunks, kRowWaves>(xrow, a.I, block * S::kChunks, chunks, rows, xs, wave, lane);
+  };
+  for (int base = blockIdx.x * (kRowWaves / 2); base < tiles; base += gridDim.x * (kRowWaves / 2)) {
+    const int tile = base + wave / 2;
+    const u32x4* src =
+        a.w + static_cast<uint64_t>(min(tile, tiles - 1)) * 2 * steps * 64 + rows::lane_chunk32(lane, h, steps);
+    rows::f32x4 acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) zero(acc[g]);
+    FirstBatch fb{};
+    __syncthreads();  // every wavefront is done with the buffers
+    stage(0, x0);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_first(src, 0, fb);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(rows::vm_wait(kBatch));
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    // Block k from `current`, block k + 1 on its way to `other`.
+    auto one = [&](int k, const uint8_t* current, uint8_t* other) {
+      const bool more = k + 1 < blocks;
+      if (more) stage(k + 1, other);
+      __builtin_amdgcn_sched_barrier(0);
+      const int n = min(kSteps, steps - k * kSteps);
+      const u32x4* at = src + static_cast<uint64_t>(k) * kSteps * 64;
+      rows::chain<G>(at, reinterpret_cast<const u32x4*>(current) + slot, 128, S::kGroup, n, acc, fb,
+                     more && steps - (k + 1) * kSteps >= kBatch ? at + kSteps * 64 : nullptr);
+      __builtin_amdgcn_sched_barrier(0);
+      // All but the next block's first weights: its inputs have landed.
+      if (fb.valid)
+        __builtin_amdgcn_s_waitcnt(rows::vm_wait(kBatch));
+      else
+        __builtin_amdgcn_s_waitcnt(rows::vm_wait(0));
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int k = 0; k < blocks; k += 2) {
+      one(k, x0, x1);
+      if (k + 1 < blocks) one(k + 1, x1, x0);
+    }
+    if (!merge_pair<G>(acc, exchange, wave, lane) || tile >= tiles) continue;
+    const float v = rows::merge<G>(acc, lane);
+    if (lane % 16 < rows)
+      residual_store(a, tile * 4 + rows::output_of(lane / 16), lane % 16, v, pos, steer, capture, steer_mask);
+  }
+}
+
+// Gate/up: a tile is [g 2j, g 2j+1, u 2j, u 2j+1]; the activations go out in
+// P32 order, the order k_rows_down stages.
+template <int R, int W>
+__global__ __launch_bounds__(W * 64) void k_rows_gateup(GateUpArgs a) {
+  using S = RowStage<R>;
+  constexpr int G = S::G;
+  __shared__ __align__(1024) uint8_t xs[S::kBytes];
+  __shared__ float scratch[W * 40];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int rows = min(a.rows, R), steps = a.D / 128, tiles = a.F / 2;
+  const int first = blockIdx.x * W + wave;
+  auto src = [&](int tile) { return a.w + static_cast<uint64_t>(tile) * steps * 64 + rows::lane_chunk16(lane); };
+  FirstBatch fb{};
+  if (!norm_rows<R, W / 2>(
+          a.h, a.norm, a.eps, StagedRows<R>{reinterpret_cast<uint16_t*>(xs), true}, scratch,
+          [&] {
+            if (first < tiles) issue_first(src(first), 0, fb);
+          },
+          &a.ctl->active, rows))
+    return;
+  __syncthreads();
+  const u32x4* x = reinterpret_cast<const u32x4*>(xs) + row_slot(lane);
+  for (int tile = first; tile < tiles; tile += gridDim.x * W) {
+    rows::f32x4 acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) zero(acc[g]);
+    const int next = tile + gridDim.x * W;
+    rows::chain<G>(src(tile), x, 64, S::kGroup, steps, acc, fb, next < tiles ? src(next) : nullptr);
+    const float v = rows::merge<G>(acc, lane);
+    // Lanes 0 .. and 32 .. hold gates 2j and 2j + 1, the next 16 their ups.
+    const float up = __shfl_down(v, 16, 64);
+    const int q = lane / 16, b = lane % 16;
+    if (q % 2 == 0 && b < rows)
+      a.act[static_cast<uint64_t>(b) * a.F + prefill::permuted(static_cast<uint32_t>(tile * 2 + q / 2), 32)] =
+          bf16_bits(silu_times(rbf(v), rbf(up)));
+  }
+}
+
+template <int R, int W>
+__global__ __launch_bounds__(W * 64) void k_rows_head(HeadArgs a) {
+  using S = RowStage<R>;
+  constexpr int G = S::G;
+  __shared__ __align__(1024) uint8_t xs[S::kBytes];
+  __shared__ float scratch[W * 40];
+  __shared__ uint64_t wave_keys[W][R];
+  __shared__ uint32_t wave_flags[W][R];
+  if (!a.ctl->active || !selecting(a.ctl)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int rows = min(a.rows, R), steps = a.D / 128, tiles = static_cast<int>(a.V / 4);
+  const int first = blockIdx.x * W + wave;
+  auto src = [&](int tile) { return a.w + static_cast<uint64_t>(tile) * steps * 64 + rows::lane_chunk16(lane); };
+  FirstBatch fb{};
+  norm_rows<R, W / 2>(
+      a.h + static_cast<uint64_t>(a.row0) * a.D, a.norm, a.eps,
+      StagedRows<R>{reinterpret_cast<uint16_t*>(xs), true}, scratch,
+      [&] {
+        if (first < tiles) issue_first(src(first), 0, fb);
+      },
+      nullptr, rows);
+  __syncthreads();
+  const u32x4* x = reinterpret_cast<const u32x4*>(xs) + row_slot(lane);
+  const int q = lane / 16, b = lane % 16;
+  uint64_t best = 0;
+  uint32_t flags = 0;
+  for (int tile = first; tile < tiles; tile += gridDim.x * W) {
+    rows::f32x4 acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) zero(acc[g]);
+    const int next = tile + gridDim.x * W;
+    rows::chain<G>(src(tile), x, 64, S::kGroup, steps, acc, fb, next < tiles ? src(next) : nullptr);
+    const float v = rows::merge<G>(acc, lane);
+    if (b < rows) {
+      const uint32_t id = static_cast<uint32_t>(tile * 4 + rows::output_of(q));
+      const uint16_t bits = bf16_bits(v);
+      a.logits[static_cast<uint64_t>(a.row0 + b) * a.V + id] = bits;
+      logit_key(bits, id, &best, &flags);
+    }
+  }
+  // Row b's keys lie in lanes 16 q + b.
+#pragma unroll
+  for (int off = 32; off >= 16; off >>= 1) {
+    const uint32_t lo = __shfl_xor(static_cast<uint32_t>(best), off);
+    const uint32_t hi = __shfl_xor(static_cast<uint32_t>(best >> 32), off);
+    const uint64_t o = (static_cast<uint64_t>(hi) << 32) | lo;
+    best = o > best ? o : best;
+    flags |= __shfl_xor(flags, off);
+  }
+  if (lane < R) {
+    wave_keys[wave][lane] = best;
+    wave_flags[wave][lane] = flags;
+  }
+  __syncthreads();
+  if (static_cast<int>(threadIdx.x) < rows) {
+    uint64_t k = 0;
+    uint32_t f = 0;
+    for (int w = 0; w < W; ++w) {
+      k = wave_keys[w][threadIdx.x] > k ? wave_keys[w][threadIdx.x] : k;
+      f |= wave_flags[w][threadIdx.x];
+    }
+    a.partial_keys[static_cast<uint64_t>(a.row0 + threadIdx.x) * gridDim.x + blockIdx.x] = k;
+    a.partial_flags[static_cast<uint64_t>(a.row0 + threadIdx.x) * gridDim.x + blockIdx.x] = f;
   }
 }
 
@@ -3387,19 +3614,21 @@ struct dl_plan {
   // Workgroups per decode-step kernel (0: one tile per wavefront).
   // Defaults from the workgroup sweep on MI355X (grid-stride over tiles).
   uint32_t grid_override[8] = {512, 0, 0, 0, 256, 768, 512, 0};
-  // The same for launches of two to four rows where the sweep differs (0:
-  // as grid_override): gate/up at 2 and 4 rows streams faster from 192
-  // workgroups than from one or three per compute unit (at 8 rows, one per
-  // compute unit, the LDS-resident count, is faster).
+  // The same for launches of two rows where the sweep differs (0: as
+  // grid_override): gate/up streams faster from 192 workgroups than from one
+  // or three per compute unit.
   uint32_t grid_override_rows[8] = {0, 0, 0, 0, 0, 192, 0, 0};
+  // The same for the kernels of three to eight rows: a workgroup per compute
+  // unit, so that none repeats the staging prologue.
+  uint32_t grid_override_many[8] = {256, 0, 0, 0, 256, 256, 256, 0};
   // Workgroups of `waves` wavefronts for `tiles` tiles of a `rows`-row
   // launch: the tuned override (or one tile per wavefront), capped at what
   // stays resident at once when the staged rows' LDS limits residency, so no
   // workgroup repeats the staging prologue in a second round.
   unsigned grid_for(int which, uint64_t tiles, size_t lds = 0, int waves = dl::kWaves, int rows = 1) const {
     const uint64_t full = dl::ceil_div(tiles, static_cast<uint64_t>(waves));
-    const bool few = rows >= 2 && rows <= 4;
-    const uint32_t tuned = few && grid_override_rows[which] ? grid_override_rows[which] : grid_override[which];
+    const uint32_t other = rows >= 3 ? grid_override_many[which] : rows == 2 ? grid_override_rows[which] : 0;
+    const uint32_t tuned = other ? other : grid_override[which];
     uint64_t g = tuned ? tuned : full;
     if (lds > 0) {
       const uint64_t resident = std::max<uint64_t>(1, dl::kLdsPerCu / (lds + 1024));
@@ -3510,39 +3739,13 @@ void allow_lds(K kernel, size_t bytes) {
                   "hipFuncSetAttribute");
 }
 
-// Largest rows per launch of each GEMV kernel: the staged FP32 inputs of
-// a row group must fit the 160 KiB LDS (QKV stages D twice, for P = 16 and
-// P = 32; down stages F = 12288 for P = 32).  Wider batches launch several
-// row groups, each streaming the weights once.
-constexpr int kQkvRows = 8;   // eight rows run as a Q launch and a K/V launch
-constexpr int kDownRows = 8;  // from four rows the inputs are staged in blocks
-constexpr int kWideRows = 8;
-
-size_t qkv_lds(int rows, int D, int part = dl::kQkvAll) {
-  const size_t q = part == dl::kQkvKV ? 0 : dl::staged_floats(16, D);
-  const size_t kv = part == dl::kQkvQ ? 0 : dl::staged_floats(32, D);
-  return size_t(rows) * (q + kv) * 4;
+// LDS of the staged FP32 inputs of the one- and two-row GEMVs (QKV stages D
+// twice, for P = 16 and P = 32).
+size_t qkv_lds(int rows, int D) {
+  return size_t(rows) * (dl::staged_floats(16, D) + dl::staged_floats(32, D)) * 4;
 }
 size_t p16_lds(int rows, int I) { return size_t(rows) * dl::staged_floats(16, I) * 4; }
 size_t p32_lds(int rows, int I) { return size_t(rows) * dl::staged_floats(32, I) * 4; }
-
-// Calls f(row0, g, rows) over row groups: `limit` rows at a time, then the
-// remaining rows as one launch of the smallest templated size g (1, 2, 4
-// or 8, at most `limit`) that holds them, whose kernels read and write only
-// its `rows` rows.  So every group streams the weights once: 3 rows run the
-// 4-row kernels, 5 to 7 rows the 8-row kernels.
-template <class F>
-void for_row_groups(uint32_t batch, int limit, F&& f) {
-  uint32_t row0 = 0;
-  while (row0 < batch) {
-    const uint32_t rest = batch - row0;
-    int g = 1;
-    while (static_cast<uint32_t>(g) < rest && g < limit) g *= 2;
-    const uint32_t rows = rest < static_cast<uint32_t>(g) ? rest : static_cast<uint32_t>(g);
-    f(row0, g, static_cast<int>(rows));
-    row0 += rows;
-  }
-}
 
 // Dynamic LDS above 64 KiB needs an explicit opt-in per kernel; this runs
 // before stream capture begins.
@@ -3554,84 +3757,69 @@ void prepare_kernels_all(dl_plan* p) {
   allow_lds(k_attn_pv_block, kPbLds);
   allow_lds(k_qkv<1>, qkv_lds(1, D));
   allow_lds(k_qkv<2>, qkv_lds(2, D));
-  allow_lds(k_qkv<4>, qkv_lds(4, D));
-  allow_lds(k_qkv_roles<8, 2>, std::max(qkv_lds(8, D, kQkvQ), qkv_lds(8, D, kQkvKV)));
-  allow_lds(k_residual_chunked<32, 4>, p32_lds(4, kChunkInputs));
-  allow_lds(k_residual_chunked<32, 8>, p32_lds(8, kChunkInputs));
   allow_lds(k_residual<16, 1>, p16_lds(1, QW));
   allow_lds(k_residual<16, 2>, p16_lds(2, QW));
-  allow_lds(k_residual<16, 4>, p16_lds(4, QW));
-  allow_lds(k_residual<16, 8, 2>, p16_lds(8, QW));
   allow_lds(k_gateup<1>, p16_lds(1, D));
   allow_lds(k_gateup<2>, p16_lds(2, D));
-  allow_lds(k_gateup<4>, p16_lds(4, D));
-  allow_lds(k_gateup<8>, p16_lds(8, D));
   allow_lds(k_residual<32, 1>, p32_lds(1, F));
   allow_lds(k_residual<32, 2>, p32_lds(2, F));
   allow_lds(k_lm_head<1>, p16_lds(1, D));
   allow_lds(k_lm_head<2>, p16_lds(2, D));
-  allow_lds(k_lm_head<4>, p16_lds(4, D));
-  allow_lds(k_lm_head<8>, p16_lds(8, D));
   allow_lds(k_attn_softmax, size_t(p->cap) * sizeof(float));
   allow_lds(k_attn_softmax_rows, size_t(p->cap) * sizeof(float));
   allow_lds(k_qkv_attn_o<2>, qkv_lds(2, D));
 }
 
-// Row groups per tile for launches with one tile per wavefront (O and the
-// split Q, K/V launches, 1024 tiles each): at eight rows two groups of four,
-// so 256 workgroups cover the chip and each chain is half as long.
-constexpr int kRowSplit(int rows, int one_tile_per_wave) { return rows == 8 && one_tile_per_wave ? 2 : 1; }
-
-template <int G, int Part = dl::kQkvAll>
+template <int G>
 void launch_qkv(dl_plan* p, hipStream_t s, const dl::QkvArgs& a) {
-  const uint64_t tiles = Part == dl::kQkvQ ? a.QW / 4 : Part == dl::kQkvKV ? a.KW : a.QW / 4 + a.KW;
-  const size_t lds = qkv_lds(G, a.D, Part);
-  constexpr int waves = dl::qkv_waves(G, Part);
-  constexpr int split = kRowSplit(G, Part == dl::kQkvAll ? 0 : 1);
-  dl::k_qkv<G, Part, split><<<p->grid_for(0, tiles * split, lds, waves), waves * 64, lds, s>>>(a);
-}
-// The Q and K/V parts of G rows as one launch (k_qkv_roles), each part with
-// the grid launch_qkv gives it.
-template <int G>
-void launch_qkv_roles(dl_plan* p, hipStream_t s, const dl::QkvArgs& a) {
-  constexpr int waves = dl::qkv_waves(G, dl::kQkvQ);
-  constexpr int split = kRowSplit(G, 1);
-  const size_t lds = std::max(qkv_lds(G, a.D, dl::kQkvQ), qkv_lds(G, a.D, dl::kQkvKV));
-  // Both parts run at once, each on half the workgroups that stay resident
-  // (measured at 8 rows: config 5 5140 -> 4952 us per step against a
-  // resident grid per part, which runs the parts one after the other; a
-  // split in proportion to the parts' weight rows, 170 + 86, 4951-4977 us).
-  const uint64_t resident = std::max<uint64_t>(2, dl::kLdsPerCu / (lds + 1024) * p->compute_units);
-  const uint64_t q_share = resident / 2, kv_share = resident - q_share;
-  const unsigned q_blocks = static_cast<unsigned>(
-      std::min<uint64_t>(q_share, p->grid_for(0, uint64_t(a.QW / 4) * split, qkv_lds(G, a.D, dl::kQkvQ), waves)));
-  const unsigned kv_blocks = static_cast<unsigned>(
-      std::min<uint64_t>(kv_share, p->grid_for(0, uint64_t(a.KW) * split, qkv_lds(G, a.D, dl::kQkvKV), waves)));
-  dl::k_qkv_roles<G, split><<<q_blocks + kv_blocks, waves * 64, lds, s>>>(a, static_cast<int>(q_blocks));
-}
-template <int G>
-void launch_down_chunked(dl_plan* p, hipStream_t s, const dl::ResidualArgs& a) {
-  const size_t lds = p32_lds(G, dl::kChunkInputs);
-  constexpr int waves = dl::gemv_waves(G);
-  dl::k_residual_chunked<32, G><<<p->grid_for(6, a.D / 2, lds, waves), waves * 64, lds, s>>>(a);
+  const size_t lds = qkv_lds(G, a.D);
+  dl::k_qkv<G><<<p->grid_for(0, a.QW / 4 + a.KW, lds), dl::kBlock, lds, s>>>(a);
 }
 template <int P, int G>
 void launch_residual(dl_plan* p, hipStream_t s, int which, const dl::ResidualArgs& a) {
   const size_t lds = P == 16 ? p16_lds(G, a.I) : p32_lds(G, a.I);
-  constexpr int split = kRowSplit(G, P == 16 ? 1 : 0);
-  dl::k_residual<P, G, split><<<p->grid_for(which, a.D / (64 / P) * split, lds, dl::gemv_waves(G)),
-                                dl::gemv_waves(G) * 64, lds, s>>>(a);
+  dl::k_residual<P, G><<<p->grid_for(which, a.D / (64 / P), lds), dl::kBlock, lds, s>>>(a);
 }
-
 template <int G>
 void launch_gateup(dl_plan* p, hipStream_t s, const dl::GateUpArgs& a) {
-  dl::k_gateup<G><<<p->grid_for(5, a.F / 2, p16_lds(G, a.D), dl::gemv_waves(G), G), dl::gemv_waves(G) * 64,
-                     p16_lds(G, a.D), s>>>(a);
+  const size_t lds = p16_lds(G, a.D);
+  dl::k_gateup<G><<<p->grid_for(5, a.F / 2, lds, dl::kWaves, G), dl::kBlock, lds, s>>>(a);
 }
 template <int G>
 void launch_head(dl_plan* p, hipStream_t s, const dl::HeadArgs& a) {
-  dl::k_lm_head<G><<<p->head_blocks, dl::gemv_waves(G) * 64, p16_lds(G, a.D), s>>>(a);
+  dl::k_lm_head<G><<<p->head_blocks, dl::kBlock, p16_lds(G, a.D), s>>>(a);
 }
+
+// The projections of three to eight rows (k_rows_*): groups of eight rows,
+// then four, the last over the rows that exist.
+template <class F>
+void for_row_tiles(uint32_t batch, F&& f) {
+  for (uint32_t row0 = 0; row0 < batch;) {
+    const uint32_t rest = batch - row0;
+    if (rest > 4) {
+      f(row0, static_cast<int>(std::min<uint32_t>(rest, 8)), std::integral_constant<int, 8>{});
+      row0 += 8;
+    } else {
+      f(row0, static_cast<int>(rest), std::integral_constant<int, 4>{});
+      row0 += 4;
+    }
+  }
+}
+
+template <int R>
+void launch_rows_qkv(dl_plan* p, hipStream_t s, const dl::QkvArgs& a) {
+  // Both parts run at once, the workgroups shared in proportion to the tiles a
+  // workgroup takes (a K/V tile takes two wavefronts, each half its chains).
+  const uint64_t q_full = dl::ceil_div(a.QW / 4, dl::kRowWaves), kv_full = dl::ceil_div(2 * a.KW / 4, dl::kRowWaves / 2);
+  const uint64_t blocks = std::max<uint64_t>(2, p->grid_for(0, (q_full + kv_full) * dl::kRowWaves, 0, dl::kRowWaves, R));
+  const uint64_t q_blocks = std::min<uint64_t>(q_full, std::max<uint64_t>(1, blocks * q_full / (q_full + kv_full)));
+  const uint64_t kv_blocks = std::min<uint64_t>(kv_full, blocks - q_blocks);
+  dl::k_rows_qkv<R><<<static_cast<unsigned>(q_blocks + kv_blocks), dl::kRowWaves * 64, 0, s>>>(
+      a, static_cast<int>(q_blocks));
+}
+
+constexpr int kRowOWaves = 4, kGateUpWaves = 8, kHeadWaves = 8;
+
 // The many-row exact GEMM: grid (output tiles, row tiles).  Each tile shape
 // leaves two workgroups per compute unit (80 and 64 KiB of LDS, 64
 // accumulators per lane), whose barriers do not fall together.  Measured for
@@ -3695,7 +3883,7 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
   const bool xg = use_xgemm(p, r);
   AttnArgs aa{ctl, r.q_raw, r.k_raw, m->q_norm[l], m->k_norm[l], p->rope, kc, vc, r.attn_seq_stride,
               r.scores, r.probs, r.att, static_cast<int>(c.q_heads), static_cast<int>(c.kv_heads),
-              static_cast<int>(p->cap), c.rms_eps, scale, r.pos_step, xg ? 1 : 0};
+              static_cast<int>(p->cap), c.rms_eps, scale, r.pos_step, B >= 3 ? 1 : 0};
   switch (which) {
     case 0:
       if (xg) {
@@ -3710,20 +3898,23 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
         launch_xgemm<32, kXgKV>(s, kva);
         break;
       }
-      for_row_groups(B, kQkvRows, [&](uint32_t r0, int g, int rows) {
-        QkvArgs qa{ctl, r.h + uint64_t(r0) * D, m->input_norm[l], reinterpret_cast<const u32x4*>(m->qkv[l]),
-                   r.q_raw + uint64_t(r0) * QW, r.k_raw + uint64_t(r0) * KW, vc + r0 * r.v_append_stride,
-                   r.v_append_stride, D, QW, KW, static_cast<int>(p->cap), c.rms_eps, rows};
-        if (g == 8) {
-          launch_qkv_roles<8>(p, s, qa);
-        } else if (g == 4) {
-          launch_qkv<4>(p, s, qa);
-        } else if (g == 2) {
+      if (B >= 3) {
+        for_row_tiles(B, [&](uint32_t r0, int rows, auto tile) {
+          launch_rows_qkv<tile.value>(
+              p, s, QkvArgs{ctl, r.h + uint64_t(r0) * D, m->input_norm[l], reinterpret_cast<const u32x4*>(m->qkv[l]),
+                            r.q_raw + uint64_t(r0) * QW, r.k_raw + uint64_t(r0) * KW, vc + r0 * r.v_append_stride,
+                            r.v_append_stride, D, QW, KW, static_cast<int>(p->cap), c.rms_eps, rows});
+        });
+        break;
+      }
+      {
+        QkvArgs qa{ctl, r.h, m->input_norm[l], reinterpret_cast<const u32x4*>(m->qkv[l]), r.q_raw, r.k_raw, vc,
+                   r.v_append_stride, D, QW, KW, static_cast<int>(p->cap), c.rms_eps, static_cast<int>(B)};
+        if (B == 2)
           launch_qkv<2>(p, s, qa);
-        } else {
+        else
           launch_qkv<1>(p, s, qa);
-        }
-      });
+      }
       break;
     case 1:
       // Consecutive positions of one sequence (their keys appended first)
@@ -3794,15 +3985,25 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
             s, XgemmArgs{ctl, r.att, oa.w, static_cast<int>(B), D, QW, nullptr, nullptr, 0, 0, 0, oa});
         break;
       }
-      for_row_groups(B, kWideRows, [&](uint32_t r0, int g, int rows) {
+      if (B >= 3) {
+        for_row_tiles(B, [&](uint32_t r0, int rows, auto tile) {
+          constexpr int R = tile.value;
+          k_rows_o<R, kRowOWaves><<<p->grid_for(4, D / 4, 0, kRowOWaves, R), kRowOWaves * 64, 0, s>>>(
+              ResidualArgs{ctl, r.att, reinterpret_cast<const u32x4*>(m->o[l]), r.h, nullptr, nullptr, QW, D,
+                           static_cast<int>(p->cap), static_cast<int>(l), static_cast<int>(r0), r.same_sequence,
+                           r.sequence, rows});
+        });
+        break;
+      }
+      {
         ResidualArgs oa{ctl, r.att, reinterpret_cast<const u32x4*>(m->o[l]), r.h, nullptr, nullptr, QW, D,
-                        static_cast<int>(p->cap), static_cast<int>(l), static_cast<int>(r0), r.same_sequence,
-                        r.sequence, rows};
-        if (g == 8) launch_residual<16, 8>(p, s, 4, oa);
-        else if (g == 4) launch_residual<16, 4>(p, s, 4, oa);
-        else if (g == 2) launch_residual<16, 2>(p, s, 4, oa);
-        else launch_residual<16, 1>(p, s, 4, oa);
-      });
+                        static_cast<int>(p->cap), static_cast<int>(l), 0, r.same_sequence, r.sequence,
+                        static_cast<int>(B)};
+        if (B == 2)
+          launch_residual<16, 2>(p, s, 4, oa);
+        else
+          launch_residual<16, 1>(p, s, 4, oa);
+      }
       break;
     case 5:
       if (xg) {
@@ -3813,14 +4014,23 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
                                                  static_cast<int>(B), 2 * F, D, r.act, nullptr, 0, 0, 0, {}});
         break;
       }
-      for_row_groups(B, kWideRows, [&](uint32_t r0, int g, int rows) {
-        GateUpArgs ga{ctl, r.h + uint64_t(r0) * D, m->post_norm[l], reinterpret_cast<const u32x4*>(m->gu[l]),
-                      r.act + uint64_t(r0) * F, D, F, c.rms_eps, rows};
-        if (g == 8) launch_gateup<8>(p, s, ga);
-        else if (g == 4) launch_gateup<4>(p, s, ga);
-        else if (g == 2) launch_gateup<2>(p, s, ga);
-        else launch_gateup<1>(p, s, ga);
-      });
+      if (B >= 3) {
+        for_row_tiles(B, [&](uint32_t r0, int rows, auto tile) {
+          constexpr int R = tile.value;
+          k_rows_gateup<R, kGateUpWaves><<<p->grid_for(5, F / 2, 0, kGateUpWaves, R), kGateUpWaves * 64, 0, s>>>(
+              GateUpArgs{ctl, r.h + uint64_t(r0) * D, m->post_norm[l], reinterpret_cast<const u32x4*>(m->gu[l]),
+                         r.act + uint64_t(r0) * F, D, F, c.rms_eps, rows});
+        });
+        break;
+      }
+      {
+        GateUpArgs ga{ctl, r.h, m->post_norm[l], reinterpret_cast<const u32x4*>(m->gu[l]), r.act, D, F, c.rms_eps,
+                      static_cast<int>(B)};
+        if (B == 2)
+          launch_gateup<2>(p, s, ga);
+        else
+          launch_gateup<1>(p, s, ga);
+      }
       break;
     case 6:
       if (xg) {
@@ -3830,27 +4040,43 @@ void launch_step_kernel(dl_plan* p, hipStream_t s, int which, uint32_t l, dl::Co
             s, XgemmArgs{ctl, r.act, da.w, static_cast<int>(B), D, F, nullptr, nullptr, 0, 0, 0, da});
         break;
       }
-      // Staging in blocks needs whole blocks of inputs; other widths keep
-      // two-row launches.
-      for_row_groups(B, F % kChunkInputs == 0 ? kDownRows : 2, [&](uint32_t r0, int g, int rows) {
+      if (B >= 3) {
+        for_row_tiles(B, [&](uint32_t r0, int rows, auto tile) {
+          constexpr int R = tile.value;
+          k_rows_down<R><<<p->grid_for(6, D / 4, 0, kRowWaves / 2, R), kRowWaves * 64, 0, s>>>(
+              ResidualArgs{ctl, r.act, reinterpret_cast<const u32x4*>(m->down[l]), r.h, p->capture, p->steer, F, D,
+                           static_cast<int>(p->cap), static_cast<int>(l), static_cast<int>(r0), r.same_sequence,
+                           r.sequence, rows});
+        });
+        break;
+      }
+      {
         ResidualArgs da{ctl, r.act, reinterpret_cast<const u32x4*>(m->down[l]), r.h, p->capture, p->steer, F, D,
-                        static_cast<int>(p->cap), static_cast<int>(l), static_cast<int>(r0), r.same_sequence,
-                        r.sequence, rows};
-        if (g == 8) launch_down_chunked<8>(p, s, da);
-        else if (g == 4) launch_down_chunked<4>(p, s, da);
-        else if (g == 2) launch_residual<32, 2>(p, s, 6, da);
-        else launch_residual<32, 1>(p, s, 6, da);
-      });
+                        static_cast<int>(p->cap), static_cast<int>(l), 0, r.same_sequence, r.sequence,
+                        static_cast<int>(B)};
+        if (B == 2)
+          launch_residual<32, 2>(p, s, 6, da);
+        else
+          launch_residual<32, 1>(p, s, 6, da);
+      }
       break;
     case 7:
-      for_row_groups(B, kWideRows, [&](uint32_t r0, int g, int rows) {
+      if (B >= 3) {
+        for_row_tiles(B, [&](uint32_t r0, int rows, auto tile) {
+          k_rows_head<tile.value, kHeadWaves><<<p->head_blocks, kHeadWaves * 64, 0, s>>>(
+              HeadArgs{ctl, r.h, m->final_norm, reinterpret_cast<const u32x4*>(m->lm_head), p->logits,
+                       p->partial_keys, p->partial_flags, D, V, c.rms_eps, static_cast<int>(r0), rows});
+        });
+        break;
+      }
+      {
         HeadArgs ha{ctl, r.h, m->final_norm, reinterpret_cast<const u32x4*>(m->lm_head), p->logits,
-                    p->partial_keys, p->partial_flags, D, V, c.rms_eps, static_cast<int>(r0), rows};
-        if (g == 8) launch_head<8>(p, s, ha);
-        else if (g == 4) launch_head<4>(p, s, ha);
-        else if (g == 2) launch_head<2>(p, s, ha);
-        else launch_head<1>(p, s, ha);
-      });
+                    p->partial_keys, p->partial_flags, D, V, c.rms_eps, 0, static_cast<int>(B)};
+        if (B == 2)
+          launch_head<2>(p, s, ha);
+        else
+          launch_head<1>(p, s, ha);
+      }
       break;
     default: fail(DL_INVALID_ARGUMENT, "unknown step kernel");
   }
@@ -4182,7 +4408,7 @@ int dl_plan_set_grid(dl_plan* plan, uint32_t which, uint32_t blocks) {
       plan->head_blocks = static_cast<int>(blocks);
     } else {
       plan->grid_override[which] = blocks;
-      plan->grid_override_rows[which] = 0;  // the value set applies at every row count
+      plan->grid_override_rows[which] = plan->grid_override_many[which] = 0;  // the value set applies at every row count
     }
     dl::check_hip(hipStreamSynchronize(plan->queue->stream), "set grid wait");
     plan->capture_step();

@@ -300,6 +300,28 @@ def test_batched_rows_follow_their_own_sequences(small_model, batch):
     assert len(streams) > 1  # the rows really differ
 
 
+@pytest.mark.parametrize("q_heads,ffn", [(12, 4352), (28, 12544)])
+@pytest.mark.parametrize("batch", [3, 7])
+def test_batched_rows_at_other_widths(device, queue, q_heads, ffn, batch):
+    """Query rows of 12 and 28 steps of 128 inputs and down rows of 17 and 49
+    steps of 256, counts that whole batches of eight steps do not divide:
+    every row equals the batch-1 run of its seed."""
+    from dolittle_amd.qwen3 import Plan, Qwen3Config, Qwen3Model, SamplingSettings
+    model = Qwen3Model(device, queue, Qwen3Config(layers=1, vocab=2048, q_heads=q_heads, kv_heads=q_heads // 4,
+                                                  ffn=ffn))
+    model.fill_synthetic(SEED + 9, 0.02)
+    settings = SamplingSettings("categorical", 1.0, 0, 0.95)
+    pb = Plan(model, batch=batch, capacity=16)
+    pb.generate([5, 900, 17], 4, settings, list(range(40, 40 + batch)))
+    tokens, _ = pb.collect()
+    for b in range(batch):
+        p1 = Plan(model, batch=1, capacity=16)
+        p1.generate([5, 900, 17], 4, settings, [40 + b])
+        assert tokens[b].tolist() == p1.collect()[0][0].tolist()
+        assert np.array_equal(pb.logits(b), p1.logits(0))
+        assert np.array_equal(pb.hidden(b), p1.hidden(0))
+
+
 @pytest.mark.parametrize("batch,grids", [
     (2, [(5, 768), (7, 256), (6, 256)]),   # gate/up, LM head and down off their 2-row defaults
     (3, [(5, 96), (4, 512)]),              # 3 rows on the 4-row kernels
