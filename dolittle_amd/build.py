@@ -19,6 +19,8 @@ BUILD = os.path.join(HERE, "_build")
 LIBRARY = os.path.join(HERE, "libdlhip.so")
 SOURCES = ["runtime.cpp", "ops.hip", "packed.hip", "qwen3.hip", "sampler.hip", "prefill.hip", "nla.hip", "sequence.hip", "archive.cpp"]
 ARCH = os.environ.get("DL_OFFLOAD_ARCH", "gfx950")
+# Device link: the kernels of these files come first and in this order.
+ORDER = {"qwen3.hip": os.path.join(CSRC, "decode_step.order")}
 
 
 def _hipcc() -> str:
@@ -43,6 +45,9 @@ def _compile(source: str) -> str:
     cmd = [_hipcc(), *_flags(), "-c", src, "-o", obj]
     if source.endswith(".cpp"):
         cmd = [_hipcc(), *_flags(), "-x", "hip", "-c", src, "-o", obj]
+    if source in ORDER:
+        for option in (f"--symbol-ordering-file={ORDER[source]}", "--fatal-warnings"):
+            cmd += ["-Xoffload-linker", option]
     result = subprocess.run(cmd, capture_output=True, text=True)
     noise = [l for l in result.stderr.splitlines() if "packed-fp32-ops" not in l and l.strip()]
     if result.returncode != 0:
