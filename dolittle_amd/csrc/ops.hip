@@ -546,7 +546,7 @@ __global__ __launch_bounds__(kRowThreads) void attention_heads(const T* __restri
   __shared__ float wave_values[kRowThreads / 64];
   __shared__ float denominator_shared;
   __shared__ float halves[2 * kHeadWidth];
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int part = tid % 8, group = tid / 8;  // 8 lanes per key, 16 features each
   const uint32_t ratio = q_heads / kv_heads;
   const uint64_t stride = static_cast<uint64_t>(kv_heads) * kHeadWidth;
@@ -560,17 +560,22 @@ __global__ __launch_bounds__(kRowThreads) void attention_heads(const T* __restri
     const T* krow = k + static_cast<uint64_t>(kvh) * kHeadWidth + 16 * part;
     float qv[16];
     load_features(q + task * kHeadWidth + 16 * part, qv);
-    constexpr int kKeys = kRowThreads / 8, kAhead = 4;
+    constexpr int kKeys = kRowThreads / 8, kAhead = sizeof(T) == 2 ? 4 : 2;
     float maximum = -INFINITY;
-    // The maximum over the thread's own scores; a NaN score is ignored, as
-    // fmaxf does in any order.
-    for (int base = 0; base < count; base += kAhead * kKeys) {
-      float kv[kAhead][16];
+    // Scores of N passes of 64 keys from `base` on, all their key rows in
+    // flight, and the maximum over the thread's own; a NaN score is ignored, as
+    // fmaxf does in any order.  `whole`: every key of the passes is visible.
+    auto pass = [&](auto n, auto whole, int base) {
+      constexpr int N = decltype(n)::value;
+      constexpr bool kWhole = decltype(whole)::value;
+      float kv[N][16];
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i)
-        load_features(krow + static_cast<uint64_t>(min(base + i * kKeys + group, count - 1)) * stride, kv[i]);
+      for (int i = 0; i < N; ++i) {
+        const int j = base + i * kKeys + group;
+        load_features(krow + static_cast<uint64_t>(kWhole ? j : min(j, count - 1)) * stride, kv[i]);
+      }
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
+      for (int i = 0; i < N; ++i) {
         const int j = base + i * kKeys + group;
         float partial = 0.0f;
 #pragma unroll
@@ -578,13 +583,30 @@ __global__ __launch_bounds__(kRowThreads) void attention_heads(const T* __restri
         partial = partial + row_down<4>(partial);
         partial = partial + row_down<2>(partial);
         partial = partial + row_down<1>(partial);
-        if (part == 0 && j < count) {
+        if (part == 0 && (kWhole || j < count)) {
           const float s = partial * scale;
           scores[j] = s;
           maximum = fmaxf(maximum, s);
         }
       }
-    }
+    };
+    // A wavefront takes no more passes than it has keys for: rows at short
+    // positions leave most slots of kAhead passes empty.  FP32 rows keep half
+    // as many in flight, the bytes of four BF16 ones: 109 registers, so two
+    // workgroups per compute unit (143 and one with four).  FP32, 32 heads,
+    // against four clamped passes throughout: 64 rows from position 0 43 -> 20
+    // us (the general kernel 27), 16 rows at 1024 keys 52 -> 39, one row at 8000
+    // 174 -> 170; BF16 within 2%, 64 rows from position 0 20 -> 17.5 us.
+    int base = 0;
+    for (; base + kAhead * kKeys <= count; base += kAhead * kKeys)
+      pass(std::integral_constant<int, kAhead>{}, std::true_type{}, base);
+    const int left = count - base - 8 * wave;  // keys from the wavefront's first on
+    if (kAhead > 2 && left > 2 * kKeys)
+      pass(std::integral_constant<int, kAhead>{}, std::false_type{}, base);
+    else if (left > kKeys)
+      pass(std::integral_constant<int, 2>{}, std::false_type{}, base);
+    else if (left > 0)
+      pass(std::integral_constant<int, 1>{}, std::false_type{}, base);
     maximum = wave_max(maximum);
     if (lane == 0) wave_values[wave] = maximum;
     __syncthreads();

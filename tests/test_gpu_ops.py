@@ -179,6 +179,41 @@ def test_attention_key_counts(device, queue, oracle, rows, first, hq, hkv):
         assert np.array_equal(down(queue, by, np.uint16, q.size), want), shift
 
 
+@pytest.mark.parametrize("rows,first", [(1, 0), (1, 7), (1, 8), (3, 14), (1, 63), (2, 64), (1, 126), (2, 127), (1, 190),
+                                        (3, 191), (1, 254), (2, 255), (1, 511), (66, 0), (1, 777)])
+@pytest.mark.parametrize("hq,hkv", [(4, 1), (3, 3)])
+def test_attention_fp32_equals_the_general_kernel(device, queue, rows, first, hq, hkv):
+    """FP32 storage: 16-byte aligned operands (the 128-feature kernel) and the
+    same operands one float further (the general kernel) give the same bits,
+    around the 8 keys of a wavefront and the passes of 64 and 128 keys; both lie
+    within FP32 rounding of the 64-bit result."""
+    width, total = 128, first + rows
+    rng = np.random.default_rng(total * 11 + hq)
+    q, k, v = (rng.standard_normal((n, width)).astype(np.float32) for n in (rows * hq, total * hkv, total * hkv))
+    scale = device.allocate(4)
+    run_op(queue, "dl_attention_scale", scale.ptr(), width)
+    got = []
+    for shift in (0, 1):
+        bq, bk, bv = (up(device, queue, np.concatenate([np.zeros(shift, np.float32), a.reshape(-1)])) for a in (q, k, v))
+        by = device.allocate(q.nbytes)
+        run_op(queue, "dl_attention", 2, bq.ptr(4 * shift), bk.ptr(4 * shift), bv.ptr(4 * shift), by.ptr(), rows, hq, hkv,
+               width, first, None, total, scale.ptr())
+        got.append(down(queue, by, np.uint32, q.size))
+    assert np.array_equal(got[0], got[1])
+    keys, values = (a.reshape(total, hkv, width).astype(np.float64) for a in (k, v))
+    out = got[0].view(np.float32).reshape(rows, hq, width)
+    for r in range(rows):
+        for h in range(hq):
+            g, n = h // (hq // hkv), first + r + 1
+            s = keys[:n, g] @ q.reshape(rows, hq, width)[r, h].astype(np.float64) / np.sqrt(width)
+            p = np.exp(s - s.max())
+            want = (p / p.sum()) @ values[:n, g]
+            # A score (19 roundings) is off by 19 * 2^-24 * sum |q k| / sqrt(width)
+            # = 1e-5 or less, so a probability by 2e-5 of itself, and the chain of
+            # up to 400 keys adds 400 * 2^-24; sum p |v| is about 1, below 2.
+            assert np.max(np.abs(out[r, h] - want)) < 1e-4
+
+
 def test_attention_reference_operands(device, queue, oracle):
     """operator_reference.cpp:273-313 shapes: 4 heads, 2 KV heads, width 128."""
     for rows in (1, 37):
