@@ -610,11 +610,10 @@ __global__ __launch_bounds__(kRowThreads) void attention_heads(const T* __restri
     maximum = wave_max(maximum);
     if (lane == 0) wave_values[wave] = maximum;
     __syncthreads();
-    // The reference starts the maximum from score 0: a row of NaN keeps it.
-    maximum = scores[0];
+    // NaN scores are ignored; if all are NaN the maximum is -infinity where the
+    // reference's is NaN, and the differences below are NaN either way.
 #pragma unroll
     for (int w = 0; w < kRowThreads / 64; ++w) maximum = fmaxf(maximum, wave_values[w]);
-    __syncthreads();
     for (int j = tid; j < count; j += kRowThreads) scores[j] = dl_expf(scores[j] - maximum);
     __syncthreads();
     if (tid < 32) {

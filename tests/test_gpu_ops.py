@@ -214,6 +214,41 @@ def test_attention_fp32_equals_the_general_kernel(device, queue, rows, first, hq
             assert np.max(np.abs(out[r, h] - want)) < 1e-4
 
 
+@pytest.mark.parametrize("code", [1, 2])
+@pytest.mark.parametrize("count", [3, 70, 300])
+def test_attention_of_nan_and_infinite_scores(device, queue, oracle, code, count):
+    """One K/V head all NaN, one with a NaN first key, one with a +infinity and
+    one with a -infinity score among ordinary ones: the 128-feature kernel (aligned
+    operands), the general kernel and, for BF16, the oracle agree."""
+    hq, hkv, width = 8, 4, 128
+    rng = np.random.default_rng(count)
+    q = np.abs(rng.standard_normal((1, hq, width))).astype(np.float32)  # the infinities' signs below are the scores'
+    k, v = (rng.standard_normal((count, hkv, width)).astype(np.float32) for _ in range(2))
+    k[:, 0, 5] = np.nan
+    k[0, 1, 7] = np.nan
+    k[count // 2, 2, 9] = np.inf
+    k[count // 2, 3, 11] = -np.inf
+    scale = device.allocate(4)
+    run_op(queue, "dl_attention_scale", scale.ptr(), width)
+    store = (lambda a: oracle.bf16_from_f32(a.reshape(-1))) if code == 1 else (lambda a: a.reshape(-1))
+    q, k, v = store(q), store(k), store(v)
+    got = []
+    for shift in (0, 1):
+        bq, bk, bv = (up(device, queue, np.concatenate([np.zeros(shift, a.dtype), a])) for a in (q, k, v))
+        by, at = device.allocate(q.nbytes), shift * q.itemsize
+        run_op(queue, "dl_attention", code, bq.ptr(at), bk.ptr(at), bv.ptr(at), by.ptr(), 1, hq, hkv, width, count - 1, None,
+               count, scale.ptr())
+        got.append(down(queue, by, q.dtype, q.size))
+    if code == 1:
+        assert np.array_equal(got[0], oracle.attention(q, k, v, 1, hq, hkv, width, count - 1))
+        assert np.array_equal(got[0], got[1])
+        got[0] = oracle.f32_from_bf16(got[0])
+    else:
+        assert np.array_equal(got[0], got[1], equal_nan=True)
+    nan = np.isnan(got[0]).reshape(hkv, -1)
+    assert nan[:3].all() and not nan[3].any()
+
+
 def test_attention_reference_operands(device, queue, oracle):
     """operator_reference.cpp:273-313 shapes: 4 heads, 2 KV heads, width 128."""
     for rows in (1, 37):
