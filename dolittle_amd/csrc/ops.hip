@@ -326,7 +326,15 @@ void launch_projection_rowmajor(hipStream_t s, const void* x, const void* w, voi
 // t+32c.  Components combine left to right, lanes reduce with shuffle-down
 // offsets 1..16, inverse = 1/sqrt(total * FP32(1/width) + eps),
 // y = round(round(x * inverse) * w).
-template <class T>
+//
+// Wide: eight loads in flight per thread, the squares still added in ascending
+// order, from the width at which a thread has eight values (1 row of 4096 BF16
+// 7.8 -> 5.3 us, 40,000 of 1000 92 -> 69).  Below it the check for a whole batch
+// only costs: 40,000 rows of 192 or 256 take 31.0 and 33.4 us without it, 32.0
+// and 35.0 with it.
+constexpr uint64_t kWideNorm = 7 * 128 + 1;
+
+template <class T, bool Wide>
 __global__ __launch_bounds__(kThreads) void rms_norm_rows(const T* __restrict__ x,
                                                           const T* __restrict__ w,
                                                           T* __restrict__ y, uint64_t rows,
@@ -345,14 +353,15 @@ __global__ __launch_bounds__(kThreads) void rms_norm_rows(const T* __restrict__ 
           comp = v * v;
         }
       } else {
-        // Eight loads in flight; the squares add in ascending order.
         uint64_t col = 4u * t + c;
-        for (; col + 7 * 128 < width; col += 8 * 128) {
-          float v[8];
+        if constexpr (Wide) {
+          for (; col + 7 * 128 < width; col += 8 * 128) {
+            float v[8];
 #pragma unroll
-          for (int k = 0; k < 8; ++k) v[k] = load_elem(xr, col + 128 * k);
+            for (int k = 0; k < 8; ++k) v[k] = load_elem(xr, col + 128 * k);
 #pragma unroll
-          for (int k = 0; k < 8; ++k) comp = comp + v[k] * v[k];
+            for (int k = 0; k < 8; ++k) comp = comp + v[k] * v[k];
+          }
         }
         for (; col < width; col += 128) {
           const float v = load_elem(xr, col);
@@ -751,14 +760,21 @@ int dl_rms_norm(dl_queue* queue, int dtype, const void* input, const void* weigh
     require(rows > 0 && width > 0, "empty normalization");
     require(epsilon > 0.0f, "epsilon must be positive");
     const unsigned grid = dl::grid_for(rows, 1, 65535);
+    auto run = [&](auto tag, auto wide) {
+      using T = decltype(tag);
+      dl::rms_norm_rows<T, decltype(wide)::value><<<grid, dl::kThreads, 0, queue->stream>>>(
+          static_cast<const T*>(input), static_cast<const T*>(weight), static_cast<T*>(output), rows, width, epsilon);
+    };
+    auto run_width = [&](auto tag) {
+      if (width >= dl::kWideNorm)
+        run(tag, std::true_type{});
+      else
+        run(tag, std::false_type{});
+    };
     if (dtype == DL_BF16)
-      dl::rms_norm_rows<uint16_t><<<grid, dl::kThreads, 0, queue->stream>>>(
-          static_cast<const uint16_t*>(input), static_cast<const uint16_t*>(weight),
-          static_cast<uint16_t*>(output), rows, width, epsilon);
+      run_width(uint16_t{});
     else
-      dl::rms_norm_rows<float><<<grid, dl::kThreads, 0, queue->stream>>>(
-          static_cast<const float*>(input), static_cast<const float*>(weight), static_cast<float*>(output),
-          rows, width, epsilon);
+      run_width(float{});
     dl::check_launch(queue, "rms_norm");
   });
 }

@@ -40,6 +40,16 @@ def test_rms_norm(device, queue, oracle, rows, width):
     assert np.array_equal(down(queue, by, np.uint16, rows * width), oracle.rms_norm(x, w, rows, width, 1e-6))
 
 
+@pytest.mark.parametrize("width", [129, 130, 895, 896, 897, 1023, 1024, 1025, 1920, 2049])
+def test_rms_norm_widths(device, queue, oracle, width):
+    """Widths around the first that batches its loads (897) and the batches' edges."""
+    rows = 3
+    x, w = oracle.operand(rows * width, 1), oracle.operand(width, 2)
+    bx, bw, by = up(device, queue, x), up(device, queue, w), device.allocate(rows * width * 2)
+    run_op(queue, "dl_rms_norm", 1, bx.ptr(), bw.ptr(), by.ptr(), rows, width, C.c_float(1e-6))
+    assert np.array_equal(down(queue, by, np.uint16, rows * width), oracle.rms_norm(x, w, rows, width, 1e-6))
+
+
 @pytest.mark.parametrize("rows,in_w,out_w", [(1, 128, 33), (1, 128, 1025), (9, 128, 33), (9, 128, 1025),
                                              (1, 4096, 4096), (1, 4096, 1024), (1, 12288, 4096), (3, 20, 1025),
                                              (2, 100, 40)])
