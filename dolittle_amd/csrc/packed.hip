@@ -154,7 +154,10 @@ int dl_projection_packed(dl_queue* queue, const void* input, const void* packed,
     const uint64_t tiles = output_width / (64 / P);
     const unsigned grid =
         static_cast<unsigned>(std::min<uint64_t>(dl::ceil_div(tiles, dl::kWaves), 2048));
-    if (rows > 1 && dl::ceil_div(rows, 16) <= 65535 && reinterpret_cast<uintptr_t>(input) % 16 == 0) {
+    // The tiles load rows and weights 16 bytes at a time straight into LDS;
+    // operands that are not 16-byte aligned go one row per launch.
+    const bool aligned = (reinterpret_cast<uintptr_t>(input) | reinterpret_cast<uintptr_t>(packed)) % 16 == 0;
+    if (rows > 1 && dl::ceil_div(rows, 16) <= 65535 && aligned) {
       dl::launch_packed_tiles(queue->stream, static_cast<const uint16_t*>(input), static_cast<const dl::u32x4*>(packed),
                               static_cast<uint16_t*>(output), rows, static_cast<int>(input_width), output_width, P,
                               output_position);

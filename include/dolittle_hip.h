@@ -172,7 +172,8 @@ int dl_gather_rows(dl_queue* queue, const void* input, void* output, uint64_t ro
  * load is a contiguous 1 KiB while the reference's partial ownership and
  * merge tree are preserved bit for bit.  Requires BF16, output_width a
  * multiple of 64/P and input_width a multiple of 8P (P from the reference's
- * rule).  The row-major weight is not modified. */
+ * rule).  The row-major weight is not modified.  Several rows run fastest from
+ * an input and packed weights that are 16-byte aligned; others are accepted. */
 int dl_projection_packed_bytes(uint64_t output_width, uint64_t input_width, uint64_t* bytes);
 int dl_projection_pack(dl_queue* queue, const void* weight, void* packed, uint64_t output_width,
                        uint64_t input_width);

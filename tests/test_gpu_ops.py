@@ -128,6 +128,22 @@ def test_projection_packed_rows(device, queue, oracle, rows, in_w, out_w):
         assert np.all(got[:2 * out_w] == 0x7fc0) and np.all(got[(rows + 2) * out_w:] == 0x7fc0)
 
 
+@pytest.mark.parametrize("rows,in_w,out_w", [(2, 128, 1028), (17, 256, 34)])
+def test_projection_packed_weights_off_alignment(device, queue, oracle, rows, in_w, out_w):
+    """Packed weights 8 bytes into an allocation: several rows give the same
+    values as weights at its start, through one row per launch."""
+    rng = np.random.default_rng(rows * 19 + out_w)
+    x = oracle.bf16_from_f32(rng.standard_normal(rows * in_w).astype(np.float32))
+    w = oracle.bf16_from_f32((0.05 * rng.standard_normal(out_w * in_w)).astype(np.float32))
+    want = oracle.projection(x, w, rows, in_w, out_w)
+    bx, bw, packed = up(device, queue, x), up(device, queue, w), device.allocate(out_w * in_w * 2 + 16)
+    for offset in (0, 8):
+        run_op(queue, "dl_projection_pack", bw.ptr(), packed.ptr(offset), out_w, in_w)
+        by = device.allocate(rows * out_w * 2)
+        run_op(queue, "dl_projection_packed", bx.ptr(), packed.ptr(offset), by.ptr(), rows, in_w, out_w, None)
+        assert np.array_equal(down(queue, by, np.uint16, rows * out_w), want), offset
+
+
 @pytest.mark.parametrize("first", [0, 1, 511, 4093, 8191])
 def test_rotary(device, queue, oracle, first):
     rows, heads, width = 3, 2, 128
