@@ -85,6 +85,20 @@ def test_exact_prefill_row_tiles(model1, rows):
     assert_same(model1, a, b, rows + 3)
 
 
+@pytest.mark.parametrize("rows", [16, 33, 97])
+@pytest.mark.parametrize("q_heads,ffn", [(12, 4352), (28, 12544)])
+def test_exact_prefill_row_tiles_at_other_widths(device, queue, q_heads, ffn, rows):
+    """Query and ffn widths that are whole stages of the many-row GEMM (128
+    and 256 inputs) but not whole 1024s: 12 and 28 stages of O inputs, 17 and
+    49 of down inputs, counts that the stage buffers do not divide."""
+    from dolittle_amd.qwen3 import Qwen3Config, Qwen3Model
+    model = Qwen3Model(device, queue, Qwen3Config(layers=2, vocab=2048, q_heads=q_heads, kv_heads=q_heads // 4, ffn=ffn))
+    model.fill_synthetic(SEED + 3, 0.02)
+    prompt = [int(t) for t in np.random.default_rng(rows + ffn).integers(0, 2048, rows + 1)]
+    a, b = run_pair(model, prompt, 2, capacity=128)
+    assert_same(model, a, b, rows + 3)
+
+
 def test_exact_prefill_across_the_fused_attention_limit(model1):
     """A 1600-id prompt: chunks below 1536 keys use the one-kernel attention,
     the later ones the split long-context kernels."""
