@@ -35,9 +35,10 @@
 namespace dl::sampling {
 
 constexpr int kBins = 65536;
-constexpr int kCountBlocks = 64;  // argmax partials a row has room for
-constexpr int kCountParts = 16;   // workgroups per row of the counting pass
-constexpr int kCountThreads = 1024;
+// Workgroups per row of the counting pass and their threads: a greedy row only
+// takes its maximum, a categorical one also counts (k_sample_count).
+constexpr int kCountBlocks = 64, kMaxThreads = 256;
+constexpr int kCountParts = 16, kCountThreads = 1024;
 constexpr int kSelectThreads = 1024;
 constexpr int kBinsPerThread = kBins / kSelectThreads;
 constexpr int kMtWords = 312;

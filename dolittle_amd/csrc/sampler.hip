@@ -186,19 +186,25 @@ __device__ __forceinline__ bool row_live(const RowsArgs& a, int row) {
 // most 65535 ids at a time, so none overflows), and adds only the values that
 // occur to the row's histogram: a 151,936-id row of a random model costs about
 // 16 x 2,500 device-scope atomics instead of one per id (48 -> 12 us; they
-// serialize where ids share a value).
-__global__ __launch_bounds__(kCountThreads) void k_sample_count(RowsArgs a) {
-  __shared__ __align__(16) uint32_t bins[kBins / 2];
-  __shared__ uint64_t wave_keys[kCountThreads / 64];
-  __shared__ uint32_t wave_flags[kCountThreads / 64];
+// serialize where ids share a value).  The 16 workgroups clear and sweep their
+// 128 KiB however short the row is, and that still costs less than the atomics:
+// one draw from 2 / 500 / 4096 ids takes 29 / 32 / 33 us, with an atomic per id
+// 39 / 76 / 87.  A greedy row counts nothing and takes no such LDS: 64 workgroups
+// of 256 threads (151,936 ids 6.7 us a selection, a million 13.0; in the counting
+// shape 7.5 and 17.5).
+template <bool Categorical>
+__global__ __launch_bounds__(Categorical ? kCountThreads : kMaxThreads) void k_sample_count(RowsArgs a) {
+  constexpr int kThreads = Categorical ? kCountThreads : kMaxThreads, kParts = Categorical ? kCountParts : kCountBlocks;
+  __shared__ __align__(16) uint32_t bins[Categorical ? kBins / 2 : 4];
+  __shared__ uint64_t wave_keys[kThreads / 64];
+  __shared__ uint32_t wave_flags[kThreads / 64];
   // Consecutive workgroups go to different XCDs; taking the row from the
   // low digit keeps each row's histogram atomics on one XCD when rows | 8.
   const int row = static_cast<int>(blockIdx.x % a.rows);
   const int part = static_cast<int>(blockIdx.x / a.rows);
   if (!row_live(a, row)) return;
-  const bool categorical = a.settings.mode == 1;
   const uint16_t* x = a.logits + static_cast<uint64_t>(row) * a.row_stride;
-  const uint32_t chunk = (a.n + kCountParts - 1) / kCountParts;
+  const uint32_t chunk = (a.n + kParts - 1) / kParts;
   const uint32_t begin = min(a.n, static_cast<uint32_t>(part) * chunk);
   const uint32_t end = min(a.n, begin + chunk);
   uint32_t* hist = a.ws.hist + static_cast<uint64_t>(row) * kBins;
@@ -209,17 +215,17 @@ __global__ __launch_bounds__(kCountThreads) void k_sample_count(RowsArgs a) {
   uint32_t flags = 0;
   for (uint32_t first = begin; first < end; first += kMost) {
     const uint32_t last = min(end, first + kMost);
-    if (categorical) {
-      for (int i = threadIdx.x; i < kQuads; i += kCountThreads) quads[i] = u32x4{0u, 0u, 0u, 0u};
+    if constexpr (Categorical) {
+      for (int i = threadIdx.x; i < kQuads; i += kThreads) quads[i] = u32x4{0u, 0u, 0u, 0u};
       __syncthreads();
     }
-    for (uint32_t base = first + threadIdx.x; base < last; base += kAhead * kCountThreads) {
+    for (uint32_t base = first + threadIdx.x; base < last; base += kAhead * kThreads) {
       uint16_t v[kAhead];
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) v[k] = x[min(base + k * kCountThreads, last - 1)];
+      for (int k = 0; k < kAhead; ++k) v[k] = x[min(base + k * kThreads, last - 1)];
 #pragma unroll
       for (int k = 0; k < kAhead; ++k) {
-        const uint32_t i = base + k * kCountThreads;
+        const uint32_t i = base + k * kThreads;
         if (i >= last) break;
         if (bf16_rejected(v[k])) {
           flags |= 1u;
@@ -228,13 +234,13 @@ __global__ __launch_bounds__(kCountThreads) void k_sample_count(RowsArgs a) {
           const uint32_t key = bf16_order(v[k]);
           const uint64_t packed = (static_cast<uint64_t>(key) << 32) | (0xffffffffu - i);
           best = packed > best ? packed : best;
-          if (categorical) atomicAdd(&bins[key / 2], (key & 1u) ? 0x10000u : 1u);
+          if constexpr (Categorical) atomicAdd(&bins[key / 2], (key & 1u) ? 0x10000u : 1u);
         }
       }
     }
-    if (categorical) {
+    if constexpr (Categorical) {
       __syncthreads();
-      for (int i = threadIdx.x; i < kQuads; i += kCountThreads) {
+      for (int i = threadIdx.x; i < kQuads; i += kThreads) {
         const u32x4 q = quads[i];
         const uint32_t words[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
@@ -255,7 +261,7 @@ __global__ __launch_bounds__(kCountThreads) void k_sample_count(RowsArgs a) {
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < kCountThreads / 64; ++w) {
+    for (int w = 1; w < kThreads / 64; ++w) {
       best = wave_keys[w] > best ? wave_keys[w] : best;
       flags |= wave_flags[w];
     }
@@ -409,7 +415,7 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
   if (tid < 64) {
     uint64_t key = 0;
     uint32_t flags = 0;
-    if (tid < kCountParts) {
+    if (tid < (categorical ? kCountParts : kCountBlocks)) {
       key = a.ws.partial_keys[static_cast<uint64_t>(row) * kCountBlocks + tid];
       flags = a.ws.partial_flags[static_cast<uint64_t>(row) * kCountBlocks + tid];
     }
@@ -739,7 +745,10 @@ Workspace carve_workspace(void* base, int rows, uint64_t vocabulary) {
 }
 
 void launch_count(hipStream_t stream, const RowsArgs& args) {
-  hipLaunchKernelGGL(k_sample_count, dim3(args.rows * kCountParts), dim3(kCountThreads), 0, stream, args);
+  if (args.settings.mode == 1)
+    hipLaunchKernelGGL(k_sample_count<true>, dim3(args.rows * kCountParts), dim3(kCountThreads), 0, stream, args);
+  else
+    hipLaunchKernelGGL(k_sample_count<false>, dim3(args.rows * kCountBlocks), dim3(kMaxThreads), 0, stream, args);
 }
 
 void launch_select(hipStream_t stream, const RowsArgs& args) {

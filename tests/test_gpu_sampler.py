@@ -294,3 +294,27 @@ def test_counting_parts_and_compaction(device, queue, oracle, kind, n):
             assert s.result() == (want, status), (top_k, top_p)
     s.submit(buf, Settings("greedy", 1.0, 0, 1.0), 0)
     assert s.result() == (int(np.argmax(logits)), 0)
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 16385, V])
+def test_greedy_and_categorical_rows_in_turn(device, queue, oracle, n):
+    """Greedy rows take 64 partial maxima, categorical ones 16: either after
+    the other sees its own only, the maximum lying in the row's last part."""
+    from dolittle_amd.sampling import Settings
+    rng = np.random.default_rng(n)
+    s = sampler(device, queue, n)
+    draws = oracle.MT19937_64(n)
+    law = Settings("categorical", 0.7, 0, 0.9)
+    for top in (50.0, 3.0, 40.0):
+        x = np.clip(rng.standard_normal(n), -4.0, 1.5).astype(np.float32)
+        x[-1] = top
+        x[n // 2] = top - 1.0
+        bits16 = bf16_bits(oracle, x)
+        logits = oracle.f32_from_bf16(bits16)
+        buf = device.upload_array(queue, bits16)
+        s.submit(buf, Settings("greedy", 1.0, 0, 1.0), 0)
+        assert s.result() == (n - 1, 0)
+        draw = draws()
+        status, want = oracle.categorical_bits(logits, 1, 0.7, 0, 0.9, draw)
+        s.submit(buf, law, draw)
+        assert s.result() == (want, status)
