@@ -12,6 +12,15 @@ namespace dl {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Operands of direct global-to-LDS loads.
+typedef __attribute__((address_space(3))) void lds_ptr;
+typedef __attribute__((address_space(1))) void global_ptr;
+
+// s_waitcnt immediate: at most n vector-memory operations outstanding (vmcnt
+// bits 3:0 and 15:14; expcnt and lgkmcnt at their no-wait maxima).
+constexpr unsigned vm_wait(unsigned n) { return 0x0f70u | (n & 0xfu) | ((n >> 4) << 14); }
 
 // Storage-typed element access: uint16_t holds BF16 bits, float is FP32.
 __device__ __forceinline__ float load_elem(const uint16_t* p, size_t i) { return dl_bf16_to_f32(p[i]); }

@@ -28,11 +28,8 @@
 
 namespace dl::exact {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x32 __attribute__((ext_vector_type(32)));
-typedef __attribute__((address_space(3))) void lds_ptr;
-typedef __attribute__((address_space(1))) void global_ptr;
 
 enum class Order { kPermuted, kNatural };
 
@@ -65,13 +62,11 @@ struct Tile {
 // workgroups and waste less on a remainder, the larger ones need fewer operand
 // reads and widenings per product.  Row-major 4096 x 12288 (16 / 32 row tiles):
 // 16 rows 31.6 / 78.5 us, 64 rows 100 / 107, 96 rows 143 / 156, 128 rows 182 /
-// 160; 12288 x 4096: 96 rows 145 / 167, 128 rows 191 / 175.
+// 160; 12288 x 4096: 96 rows 145 / 167, 128 rows 191 / 175.  (The 32-row
+// natural-order tiles measured spill 30 and 40 registers: see k_project_tiles.)
 constexpr uint64_t kTileFewRows = 96;
 
-// s_waitcnt immediates: at most n vector-memory operations outstanding (vmcnt
-// bits 3:0 and 15:14; expcnt and lgkmcnt at their no-wait maxima); the same
-// and no LDS operation outstanding.
-constexpr unsigned vm_wait(unsigned n) { return 0x0f70u | (n & 0xfu) | ((n >> 4) << 14); }
+// vm_wait with no LDS operation outstanding either.
 constexpr unsigned vm_lds_wait(unsigned n) { return 0x0070u | (n & 0xfu) | ((n >> 4) << 14); }
 
 // A lane's operands of one tile for half a group (chain steps 4 half .. + 3):

@@ -202,10 +202,9 @@ __device__ __forceinline__ void chain_tile_pipelined(const u32x4* __restrict__ s
   }
 }
 
-// The chain steps of one tile over I staged inputs, accumulating into acc
-// (not reset).  `next` (optional) is where the wavefront's chain continues
-// (its next tile, or this tile's next block of inputs): with B >= 2 its
-// first batch is loaded during this call's last batch and left in `first`.
+// The chain steps of one tile over I staged inputs, accumulating into acc.
+// `next` (optional) is the wavefront's next tile: with kDeep its first batch is
+// loaded during this call's last batch and left in `first`.
 // kDeep selects the double-buffered batches (the default for B >= 2; a
 // single-row caller that leaves few wavefronts per SIMD asks for it too, to
 // keep two batches in flight per wavefront).
@@ -267,40 +266,10 @@ __device__ __forceinline__ void chain_tile(const u32x4* __restrict__ tile, const
   chain_merge<P, B>(acc);
 }
 
-// Inverse RMS of one BF16 row of width D > 128 with the reference tree
-// (normalization.cu:134-186): thread i < 128 owns component sum i of
-// features i + 128k, groups of four combine left to right, 32 lane totals
-// reduce with shuffle-down offsets 1..16.  Every thread of the block calls;
-// `scratch` holds at least 33 floats of LDS.  Returns the inverse to all.
-__device__ __forceinline__ float block_rms_inverse(const uint16_t* __restrict__ x, int D, float eps,
-                                                   float* scratch) {
-  const int tid = threadIdx.x;
-  if (tid < 128) {
-    float comp = 0.0f;
-    for (int col = tid; col < D; col += 128) {
-      const float v = dl_bf16_to_f32(x[col]);
-      comp = comp + v * v;
-    }
-    const float second = row_down<1>(comp);
-    const float third = row_down<2>(comp);
-    const float fourth = row_down<3>(comp);
-    if ((tid & 3) == 0) scratch[tid >> 2] = ((comp + second) + third) + fourth;
-  }
-  __syncthreads();
-  if (tid < 32) {
-    const float s = tree_sum32(scratch[tid]);
-    if (tid == 0) scratch[32] = inverse_sqrt(s * (1.0f / static_cast<float>(D)) + eps);
-  }
-  __syncthreads();
-  const float inverse = scratch[32];
-  __syncthreads();
-  return inverse;
-}
-
 // to.put(b, i, v) with v = round(round(h_b * inverse_b) * gain) for the rows
 // [b0, b0 + R G) that exist (below B) of width D = 128 * kNormK, computing
-// inverse_b with the reference tree (normalization.cu:134-186) in the same pass.  Thread group
-// g (threads 128 g .. 128 g + 127) owns rows b0 + R g .. b0 + R g + R - 1:
+// inverse_b with the reference tree (normalization.cu:134-186) in the same
+// pass.  Thread group g (threads 128 g .. 128 g + 127) owns rows b0 + R g .. b0 + R g + R - 1:
 // thread t of the group keeps features t + 128k of its rows in registers, sums
 // their squares in ascending k (component t), combines groups of four left
 // to right, and the group's first wavefront reduces the 32 lane totals of
@@ -376,9 +345,9 @@ __device__ __forceinline__ bool norm_rows_pass(const uint16_t* __restrict__ h, c
 // G groups cover the B rows in one pass, else 2) (scratch is reused between
 // passes behind a barrier); G = threads / 128 of the calling workgroup.
 // Rows have width kNormWidth; to.put(row, column, value) stores each
-// normalized value.  Returns false, before any math, when the loop word `active` (read in
-// the first pass, as in stage_rows) is zero.  Only the first `rows` (at most
-// B) rows exist and are read and stored.
+// normalized value.  Returns false, before any math, when the loop word
+// `active` (read in the first pass, as in stage_rows) is zero.  Only the first
+// `rows` (at most B) rows exist and are read and stored.
 template <int B, int G, class To, class Issue>
 __device__ __forceinline__ bool norm_rows(const uint16_t* __restrict__ h, const uint16_t* __restrict__ gain, float eps,
                                           const To& to, float* scratch, Issue&& issue, const uint32_t* active,

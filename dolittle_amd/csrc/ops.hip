@@ -80,11 +80,17 @@ __global__ __launch_bounds__(kThreads) void projection_rowmajor(const T* __restr
 // rows are bound by the weight stream (16 rows of 4096 x 12288: 31 us, 3.2
 // TB/s; 384 us with one lane per partial reading 2 bytes at a time), many by
 // the FP32 MFMA rate and the operand widening.
+//
+// Wavefronts per SIMD, which bound the registers: the 32-row tiles (eight
+// wavefronts, 64 and 80 KiB of LDS) are held at two workgroups per compute
+// unit, 128 registers, and spill 30 (P = 16) and 40 (P = 32) of them to
+// scratch inside the loop; the 16-row tiles take what their LDS leaves room
+// for, two workgroups of four wavefronts (P = 16) or of eight (P = 32), and do
+// not spill.
 template <class T>
-__global__ __launch_bounds__(T::kThreads) __attribute__((amdgpu_waves_per_eu(T::Edge == 32 ? 4 : T::P / 8))) void k_project_tiles(const uint16_t* __restrict__ x,
-                                                               const uint16_t* __restrict__ w,
-                                                               uint16_t* __restrict__ y, uint64_t rows, uint64_t in_w,
-                                                               uint64_t out_w, const uint64_t* out_pos) {
+__global__ __launch_bounds__(T::kThreads) __attribute__((amdgpu_waves_per_eu(T::Edge == 32 ? 4 : T::P / 8)))
+void k_project_tiles(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
+                     uint64_t rows, uint64_t in_w, uint64_t out_w, const uint64_t* out_pos) {
   const uint64_t id = blockIdx.x + static_cast<uint64_t>(blockIdx.y) * gridDim.x;
   // XCD x takes the output tiles x, x + 8, ..., all row tiles of one together.
   const bool by_xcd = gridDim.x % 8 == 0;
@@ -100,7 +106,7 @@ __global__ __launch_bounds__(T::kThreads) __attribute__((amdgpu_waves_per_eu(T::
       [&](int row, int piece) {
         return reinterpret_cast<const u32x4*>(x + min(r0 + row, rows - 1) * in_w) + piece;
       },
-      [&](int output, int row, exact::f32x4 sum) {
+      [&](int output, int row, f32x4 sum) {
         const uint64_t r = r0 + row, o = o0 + output;
         if (r >= rows || o >= out_w) return;
         uint16_t v[4];
@@ -181,8 +187,8 @@ __global__ __launch_bounds__(T::kThreads) void k_project_row(const uint16_t* __r
   auto issue = [&](int s, uint8_t* buffer) {
 #pragma unroll
     for (int i = 0; i < T::kLoads; ++i)
-      __builtin_amdgcn_global_load_lds((const exact::global_ptr*)(src[i] + static_cast<uint64_t>(s) * T::kRowBytes),
-                                       (exact::lds_ptr*)(buffer + i * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const global_ptr*)(src[i] + static_cast<uint64_t>(s) * T::kRowBytes),
+                                       (lds_ptr*)(buffer + i * 1024), 16, 0, 0);
   };
   for_each_index(std::make_integer_sequence<int, T::kRing>{}, [&](auto i) {
     issue(min(static_cast<int>(i.value), stages - 1), row_stage<T, i.value>(wave));
@@ -203,7 +209,7 @@ __global__ __launch_bounds__(T::kThreads) void k_project_row(const uint16_t* __r
 #pragma unroll
   for (int i = 0; i < C; ++i) acc[i] = 0.0f;
   auto one = [&](int s, uint8_t* buffer) {
-    __builtin_amdgcn_s_waitcnt(exact::vm_wait((T::kRing - 1) * T::kLoads));  // stage s has landed
+    __builtin_amdgcn_s_waitcnt(vm_wait((T::kRing - 1) * T::kLoads));  // stage s has landed
     __builtin_amdgcn_sched_barrier(0);
     const uint8_t* row = buffer + r * T::kRowBytes;
     const float* xt = xs + s * T::kInputs + C * j;
@@ -235,7 +241,7 @@ __global__ __launch_bounds__(T::kThreads) void k_project_row(const uint16_t* __r
       if (s + i.value < stages) one(s + i.value, row_stage<T, i.value>(wave));
     });
   }
-  __builtin_amdgcn_s_waitcnt(exact::vm_wait(0));  // no load outlives the wavefront
+  __builtin_amdgcn_s_waitcnt(vm_wait(0));  // no load outlives the wavefront
 
   // Offsets P / 2 .. C across the output's lanes, the rest within the lane.
 #pragma unroll

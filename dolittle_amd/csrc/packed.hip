@@ -78,7 +78,7 @@ __global__ __launch_bounds__(T::kThreads) void k_packed_tiles(const uint16_t* __
       [&](int row, int piece) {
         return reinterpret_cast<const u32x4*>(x + min(r0 + row, rows - 1) * in_w) + piece;
       },
-      [&](int output, int row, exact::f32x4 sum) {
+      [&](int output, int row, f32x4 sum) {
         if (r0 + row >= rows) return;
 #pragma unroll
         for (int i = 0; i < 4; ++i)

@@ -2420,7 +2420,7 @@ __global__ __launch_bounds__(T::kThreads) __attribute__((amdgpu_waves_per_eu(4))
       [&](int row, int piece) {
         return reinterpret_cast<const u32x4*>(a.x + static_cast<uint64_t>(min(b0 + row, a.B - 1)) * a.K) + piece;
       },
-      [&](int output, int row, exact::f32x4 sum) {
+      [&](int output, int row, f32x4 sum) {
         const int b = b0 + row, f = f0 + output;
         if (b >= a.B) return;
         if constexpr (EPI == kXgGateUp) {
@@ -2610,14 +2610,14 @@ struct StagedRows {
 // The wavefront's slot in every piece (rows::slot_of for its partial and row).
 __device__ __forceinline__ int row_slot(int lane) { return rows::slot_of(lane / 4, lane % 4); }
 
-__device__ __forceinline__ void zero(rows::f32x4& v) { v = rows::f32x4{0.0f, 0.0f, 0.0f, 0.0f}; }
+__device__ __forceinline__ void zero(f32x4& v) { v = f32x4{0.0f, 0.0f, 0.0f, 0.0f}; }
 
 // Two wavefronts share a P = 32 tile, each with 16 partials (h = 0, 1): offset
 // 16 across them through `exchange` ([pair][G][64]).  Every wavefront of the
 // workgroup calls; true where the sums are (h = 0).
 template <int G>
-__device__ __forceinline__ bool merge_pair(rows::f32x4 (&acc)[G], rows::f32x4* exchange, int wave, int lane) {
-  rows::f32x4* at = exchange + (wave / 2) * G * 64 + lane;
+__device__ __forceinline__ bool merge_pair(f32x4 (&acc)[G], f32x4* exchange, int wave, int lane) {
+  f32x4* at = exchange + (wave / 2) * G * 64 + lane;
   __syncthreads();
   if (wave % 2) {
 #pragma unroll
@@ -2627,7 +2627,7 @@ __device__ __forceinline__ bool merge_pair(rows::f32x4 (&acc)[G], rows::f32x4* e
   if (wave % 2) return false;
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    const rows::f32x4 upper = at[g * 64];
+    const f32x4 upper = at[g * 64];
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[g][i] = acc[g][i] + upper[i];
   }
@@ -2642,7 +2642,7 @@ __global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(
   using S = RowStage<R>;
   constexpr int G = S::G;
   __shared__ __align__(1024) uint8_t xs[S::kBytes];
-  __shared__ rows::f32x4 exchange[kRowWaves / 2 * G * 64];
+  __shared__ f32x4 exchange[kRowWaves / 2 * G * 64];
   __shared__ float scratch[kRowWaves * 40];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const bool q_part = static_cast<int>(blockIdx.x) < q_blocks;
@@ -2674,7 +2674,7 @@ __global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(
   const int q = lane / 16, b = lane % 16;
   if (q_part) {
     for (int tile = first; tile < tiles; tile += blocks * per_block) {
-      rows::f32x4 acc[G];
+      f32x4 acc[G];
 #pragma unroll
       for (int g = 0; g < G; ++g) zero(acc[g]);
       const int next = tile + blocks * per_block;
@@ -2686,7 +2686,7 @@ __global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(
   }
   for (int base = block * per_block; base < tiles; base += blocks * per_block) {
     const int tile = base + wave / 2, next = tile + blocks * per_block;
-    rows::f32x4 acc[G];
+    f32x4 acc[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) zero(acc[g]);
     if (tile < tiles)
@@ -2721,13 +2721,13 @@ __global__ __launch_bounds__(Waves * 64) void k_rows_o(ResidualArgs a) {
   if (first < tiles) issue_first(src(first), 0, fb);
   __builtin_amdgcn_sched_barrier(0);
   if (!live) {
-    __builtin_amdgcn_s_waitcnt(rows::vm_wait(0));  // no load outlives the workgroup
+    __builtin_amdgcn_s_waitcnt(vm_wait(0));  // no load outlives the workgroup
     return;
   }
   if (first < tiles)
-    __builtin_amdgcn_s_waitcnt(rows::vm_wait(kBatch));  // the staged rows, issued before the weights
+    __builtin_amdgcn_s_waitcnt(vm_wait(kBatch));  // the staged rows, issued before the weights
   else
-    __builtin_amdgcn_s_waitcnt(rows::vm_wait(0));
+    __builtin_amdgcn_s_waitcnt(vm_wait(0));
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
   const uint64_t pos = a.ctl->position;
@@ -2736,7 +2736,7 @@ __global__ __launch_bounds__(Waves * 64) void k_rows_o(ResidualArgs a) {
   const uint32_t steer_mask = a.ctl->steer_mask;
   const u32x4* x = reinterpret_cast<const u32x4*>(xs) + row_slot(lane);
   for (int tile = first; tile < tiles; tile += gridDim.x * Waves) {
-    rows::f32x4 acc[G];
+    f32x4 acc[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) zero(acc[g]);
     const int next = tile + gridDim.x * Waves;
@@ -2754,7 +2754,7 @@ __global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(
   using S = RowStage<R>;
   constexpr int G = S::G, kSteps = S::kChunks / 2;
   __shared__ __align__(1024) uint8_t x0[S::kBytes], x1[S::kBytes];
-  __shared__ rows::f32x4 exchange[kRowWaves / 2 * G * 64];
+  __shared__ f32x4 exchange[kRowWaves / 2 * G * 64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int h = wave % 2, rows = min(a.rows, R);
   const int steps = a.I / 256, chunks = a.I / 128, blocks = (steps + kSteps - 1) / kSteps, tiles = a.D / 4;
@@ -2772,7 +2772,7 @@ __global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(
     const int tile = base + wave / 2;
     const u32x4* src =
         a.w + static_cast<uint64_t>(min(tile, tiles - 1)) * 2 * steps * 64 + rows::lane_chunk32(lane, h, steps);
-    rows::f32x4 acc[G];
+    f32x4 acc[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) zero(acc[g]);
     FirstBatch fb{};
@@ -2781,7 +2781,7 @@ __global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(
     __builtin_amdgcn_sched_barrier(0);
     issue_first(src, 0, fb);
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(rows::vm_wait(kBatch));
+    __builtin_amdgcn_s_waitcnt(vm_wait(kBatch));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     // Block k from `current`, block k + 1 on its way to `other`.
@@ -2796,9 +2796,9 @@ __global__ __launch_bounds__(kRowWaves * 64) __attribute__((amdgpu_waves_per_eu(
       __builtin_amdgcn_sched_barrier(0);
       // All but the next block's first weights: its inputs have landed.
       if (fb.valid)
-        __builtin_amdgcn_s_waitcnt(rows::vm_wait(kBatch));
+        __builtin_amdgcn_s_waitcnt(vm_wait(kBatch));
       else
-        __builtin_amdgcn_s_waitcnt(rows::vm_wait(0));
+        __builtin_amdgcn_s_waitcnt(vm_wait(0));
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
     };
@@ -2836,7 +2836,7 @@ __global__ __launch_bounds__(W * 64) void k_rows_gateup(GateUpArgs a) {
   __syncthreads();
   const u32x4* x = reinterpret_cast<const u32x4*>(xs) + row_slot(lane);
   for (int tile = first; tile < tiles; tile += gridDim.x * W) {
-    rows::f32x4 acc[G];
+    f32x4 acc[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) zero(acc[g]);
     const int next = tile + gridDim.x * W;
@@ -2878,7 +2878,7 @@ __global__ __launch_bounds__(W * 64) void k_rows_head(HeadArgs a) {
   uint64_t best = 0;
   uint32_t flags = 0;
   for (int tile = first; tile < tiles; tile += gridDim.x * W) {
-    rows::f32x4 acc[G];
+    f32x4 acc[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) zero(acc[g]);
     const int next = tile + gridDim.x * W;

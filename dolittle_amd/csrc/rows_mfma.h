@@ -26,12 +26,6 @@
 
 namespace dl::rows {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_ptr;
-typedef __attribute__((address_space(1))) void global_ptr;
-
-constexpr unsigned vm_wait(unsigned n) { return 0x0f70u | (n & 0xfu) | ((n >> 4) << 14); }
-
 // 16-byte slot of partial t (below 16) of row j (below 4) in its piece.
 __device__ __forceinline__ int slot_of(int t, int j) { return 4 * t + (j ^ (t / 4)); }
 

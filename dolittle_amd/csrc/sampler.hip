@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
   __shared__ Found s_found[4];
   __shared__ uint32_t s_token;
   __shared__ uint32_t s_pick[2];
-  __shared__ uint64_t s_scan[kSelectThreads / 64];
+  __shared__ uint32_t s_scan[kSelectThreads / 64];
   __shared__ uint16_t s_keys[kBins];  // the distinct values' keys, descending
 
   const int row = blockIdx.x;
@@ -610,7 +610,7 @@ __global__ __launch_bounds__(kSelectThreads) void k_sample_select(RowsArgs a) {
     if (lane == 0) s_scan[wave] = hits;
     __syncthreads();
     for (int w = 0; w < wave; ++w) {
-      const uint32_t earlier = static_cast<uint32_t>(s_scan[w]);
+      const uint32_t earlier = s_scan[w];
       wanted = wanted > earlier ? wanted - earlier : 0u;
       if (wanted == 0) break;  // in an earlier part
     }

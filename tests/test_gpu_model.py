@@ -254,10 +254,10 @@ def test_batch_two_equals_batch_one(small_model):
 
 
 def test_batch_eight_equals_batch_one(small_model):
-    """Batch 8 runs Q and K/V as two launches, the down projection with its
-    inputs staged in 4096-wide blocks, and the 8-row gate/up, O and LM-head
-    kernels; every sequence reproduces the batch-1 stream and its last
-    logits bit for bit."""
+    """Batch 8 runs the 8-row kernels: Q and K/V workgroups in one launch, O,
+    gate/up, the down projection with its inputs staged in 4096-wide blocks,
+    and the LM head; every sequence reproduces the batch-1 stream and its
+    last logits bit for bit."""
     from dolittle_amd.qwen3 import Plan
     prompt = [9, 150000, 3, 77, 4096]
     p1 = Plan(small_model, batch=1, capacity=32)
